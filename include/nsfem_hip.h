@@ -218,12 +218,17 @@ int nsfem_solver_set_mse_check_interval(nsfem_solver * s, int interval);
  *                  scaled to (G M G^T)_ii = 1, built on the host when first
  *                  chosen: two parallel launches per application instead of
  *                  2 colours - 2 dependent sweeps (the P2 mass matrix: 12
- *                  iterations where GS takes 13).
+ *                  iterations where GS takes 13).  Its solves run on a copy
+ *                  of the system in locality order; with fused reductions and
+ *                  1 or 2 channels on slices of 64 rows with a launch shape
+ *                  of their own, so the row counts and lanes of the options
+ *                  above (and autotune's) do not reach their kernels.
  *   "rowsPreconditioner" fused reductions on one system, preconditioner
  *                  1: rows per workgroup of the approximate inverse's two
  *                  launches on a region-major map of their own (a positive
  *                  multiple of 256); 0 (default) shares the direction
- *                  kernel's map.
+ *                  kernel's map.  Accepted without effect on 1 and 2
+ *                  channels, whose launches run on slices of 64 rows.
  *   "amgChebyshevFrom", "amgChebyshevDegree", "amgChebyshevFraction"
  *                  amg_pcg: the V-cycle levels from this one on (but the
  *                  dense coarsest) are smoothed by this many steps of the

@@ -587,12 +587,12 @@ namespace nsfem
 
     // Registers of the fused reductions' loads (fusedRhoLoad / fusedRhoFinish).
     constexpr int kFusedPre = 8;
-    template <int NCH>
+    template <int NCH, int BLOCK = kBlock, int PRE = kFusedPre>
     struct FusedRhoLoads
     {
         int first, was;
         double ref, rhoOld;
-        double rho[kFusedPre], rr[kFusedPre];
+        double rho[PRE], rr[PRE];
     };
 
     // Finishes a per-system reduction in a one-block finalize kernel of
@@ -1258,8 +1258,8 @@ namespace nsfem
     // Block sum per channel when every thread holds one channel's value,
     // channel = threadIdx.x % NCH (lanes of one channel are NCH apart in a
     // wavefront).  The total of channel c is returned in thread c (c < NCH).
-    template <int NCH>
-    __device__ __forceinline__ double channelBlockSum(double v, double * sm /* NCH * kWaves */)
+    template <int NCH, int W = kWaves>
+    __device__ __forceinline__ double channelBlockSum(double v, double * sm /* NCH * W */)
     {
 #pragma unroll
         for (int off = 32; off >= NCH; off >>= 1)
@@ -1270,16 +1270,16 @@ namespace nsfem
         const int lane = threadIdx.x & 63;
         if (lane < NCH)
         {
-            sm[lane * kWaves + wave] = v;
+            sm[lane * W + wave] = v;
         }
         __syncthreads();
         double s = 0;
         if (static_cast<int>(threadIdx.x) < NCH)
         {
 #pragma unroll
-            for (int w = 0; w < kWaves; w++)
+            for (int w = 0; w < W; w++)
             {
-                s += sm[threadIdx.x * kWaves + w];
+                s += sm[threadIdx.x * W + w];
             }
         }
         __syncthreads();
@@ -1287,8 +1287,8 @@ namespace nsfem
     }
 
     // channelBlockSum of two values at once (one pair of barriers); sm holds
-    // 2 * NCH * kWaves doubles.  Totals in threads c < NCH.
-    template <int NCH>
+    // 2 * NCH * W doubles.  Totals in threads c < NCH.
+    template <int NCH, int W = kWaves>
     __device__ __forceinline__ void channelBlockSum2(double & a, double & b, double * sm)
     {
 #pragma unroll
@@ -1301,18 +1301,18 @@ namespace nsfem
         const int lane = threadIdx.x & 63;
         if (lane < NCH)
         {
-            sm[lane * kWaves + wave] = a;
-            sm[(NCH + lane) * kWaves + wave] = b;
+            sm[lane * W + wave] = a;
+            sm[(NCH + lane) * W + wave] = b;
         }
         __syncthreads();
         double sa = 0, sb = 0;
         if (static_cast<int>(threadIdx.x) < NCH)
         {
 #pragma unroll
-            for (int w = 0; w < kWaves; w++)
+            for (int w = 0; w < W; w++)
             {
-                sa += sm[threadIdx.x * kWaves + w];
-                sb += sm[(NCH + threadIdx.x) * kWaves + w];
+                sa += sm[threadIdx.x * W + w];
+                sb += sm[(NCH + threadIdx.x) * W + w];
             }
         }
         __syncthreads();
@@ -1348,10 +1348,10 @@ namespace nsfem
     }
 
     // Fused reductions, first half: the flags, the system's per-channel state
-    // and up to kFusedPre partial sums per thread of each set load into
+    // and up to PRE partial sums per thread of each set load into
     // registers, so that they are in flight with the kernel's first row loads.
-    template <int NCH>
-    __device__ __forceinline__ void fusedRhoLoad(const SolveState & st, const FusedSlice & sl, FusedRhoLoads<NCH> & f)
+    template <int NCH, int BLOCK = kBlock, int PRE = kFusedPre>
+    __device__ __forceinline__ void fusedRhoLoad(const SolveState & st, const FusedSlice & sl, FusedRhoLoads<NCH, BLOCK, PRE> & f)
     {
         const int t = static_cast<int>(threadIdx.x);
         f.first = st.flags[1];
@@ -1365,13 +1365,13 @@ namespace nsfem
             f.ref = st.ref[k];
             f.rhoOld = st.rho[k];
         }
-        constexpr int G = kBlock / NCH; // threads per channel
+        constexpr int G = BLOCK / NCH; // threads per channel
         const int c = t % NCH;
         const int i0 = t / NCH;
         const double * pr = st.partials + static_cast<size_t>(sl.base) * NCH;
         const double * pu = st.partials2 + static_cast<size_t>(sl.base) * NCH;
 #pragma unroll
-        for (int k = 0; k < kFusedPre; k++)
+        for (int k = 0; k < PRE; k++)
         {
             const int i = i0 + k * G;
             f.rho[k] = i < sl.rhoParts ? pr[static_cast<size_t>(i) * NCH + c] : 0.0;
@@ -1389,32 +1389,32 @@ namespace nsfem
     // results for the host; no block of this launch reads those.  Returns
     // whether any channel of the system goes on; beta and activity per
     // channel in LDS.
-    template <int NCH>
-    __device__ __forceinline__ bool fusedRhoFinish(const SolveState & st, const FusedRhoLoads<NCH> & f, const FusedSlice & sl,
+    template <int NCH, int BLOCK = kBlock, int PRE = kFusedPre>
+    __device__ __forceinline__ bool fusedRhoFinish(const SolveState & st, const FusedRhoLoads<NCH, BLOCK, PRE> & f, const FusedSlice & sl,
                                                    double * sm, double * shBeta, int * shAct)
     {
         const int t = static_cast<int>(threadIdx.x);
-        constexpr int G = kBlock / NCH;
+        constexpr int G = BLOCK / NCH;
         const int c = t % NCH;
         double rho = 0, rr = 0;
 #pragma unroll
-        for (int k = 0; k < kFusedPre; k++)
+        for (int k = 0; k < PRE; k++)
         {
             rho += f.rho[k];
             rr += f.rr[k];
         }
-        // beyond the preloaded slots (more than kFusedPre * G partials)
+        // beyond the preloaded slots (more than PRE * G partials)
         const double * pr = st.partials + static_cast<size_t>(sl.base) * NCH;
         const double * pu = st.partials2 + static_cast<size_t>(sl.base) * NCH;
-        for (int i = t / NCH + kFusedPre * G; i < sl.rhoParts; i += G)
+        for (int i = t / NCH + PRE * G; i < sl.rhoParts; i += G)
         {
             rho += pr[static_cast<size_t>(i) * NCH + c];
         }
-        for (int i = t / NCH + kFusedPre * G; i < sl.updParts; i += G)
+        for (int i = t / NCH + PRE * G; i < sl.updParts; i += G)
         {
             rr += pu[static_cast<size_t>(i) * NCH + c];
         }
-        channelBlockSum2<NCH>(rho, rr, sm);
+        channelBlockSum2<NCH, BLOCK / 64>(rho, rr, sm);
         const int first = f.first;
         if (t < NCH)
         {

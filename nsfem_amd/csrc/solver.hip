@@ -587,7 +587,8 @@ namespace nsfem
 
     // Workgroups of at most rpb rows, colour-major, never straddling a
     // (colour, system) chunk; colorStart[c] = first workgroup of colour c.
-    void McgsSolver::buildBlocks(int rpb, std::vector<int4> & blocks, std::vector<int> & blockSystem, std::vector<int> & colorStart) const
+    void McgsSolver::buildBlocks(const std::vector<RowChunk> & chunks, int rpb, std::vector<int4> & blocks, std::vector<int> & blockSystem,
+                                 std::vector<int> & colorStart) const
     {
         blocks.clear();
         blockSystem.clear();
@@ -596,9 +597,9 @@ namespace nsfem
         for (int c = 0; c < numColors_; c++)
         {
             colorStart[c] = static_cast<int>(blocks.size());
-            for (; next < chunks_.size() && chunks_[next].color == c; next++)
+            for (; next < chunks.size() && chunks[next].color == c; next++)
             {
-                const RowChunk & ch = chunks_[next];
+                const RowChunk & ch = chunks[next];
                 for (int b0 = ch.begin; b0 < ch.end; b0 += rpb)
                 {
                     blocks.push_back(int4{b0, std::min(ch.end, b0 + rpb), ch.system, -1});
@@ -617,7 +618,7 @@ namespace nsfem
         sweepRows_ = rpb;
         std::vector<int4> blocks;
         std::vector<int> blockSystem;
-        buildBlocks(rpb, blocks, blockSystem, colorSweepBlockStart_);
+        buildBlocks(chunks_, rpb, blocks, blockSystem, colorSweepBlockStart_);
         sweepBlocks_.upload(blocks.empty() ? std::vector<int4>{int4{0, 0, 0, 0}} : blocks);
         sweepBm_ = bm_;
         sweepBm_.blocks = sweepBlocks_.get();
@@ -645,7 +646,20 @@ namespace nsfem
         NSFEM_HIP(hipStreamSynchronize(stream_));
         lanes_ = L;
         rowsPerBlock_ = rpb;
+        setupMainMap();
 
+        // reduction scratch sized by the block count; captured graphs hold
+        // the old launch shapes and buffers
+        rowsDir_ = rowsUpd_ = rowsRho_ = 0;
+        lanesDir_ = 0;
+        setupKindMaps();
+        // the sweeps take the same shape until reshapeSweeps
+        reshapeSweeps(lanes_, rowsPerBlock_);
+    }
+
+    void McgsSolver::setupMainMap()
+    {
+        const int rpb = rowsPerBlock_;
         std::vector<int4> blocks;
         std::vector<int> blockSystem;
         if (flat())
@@ -662,7 +676,7 @@ namespace nsfem
         else
         {
             std::vector<int> colorStart;
-            buildBlocks(rpb, blocks, blockSystem, colorStart);
+            buildBlocks(local() ? loc_.chunks : chunks_, rpb, blocks, blockSystem, colorStart);
             color0Blocks_ = colorStart.size() > 1 ? colorStart[1] : 0;
         }
         numBlocks_ = static_cast<int>(blocks.size());
@@ -689,14 +703,6 @@ namespace nsfem
         sysBlocks_.upload(sysBlocks.empty() ? std::vector<int>{0} : sysBlocks);
         bm_ = BlockMap{blocks_.get(), sysBlockStart_.get(), sysBlocks_.get(), systemRows_.get(), numSystems_, numBlocks_,
                        flat() ? n_ : 0, rpb};
-
-        // reduction scratch sized by the block count; captured graphs hold
-        // the old launch shapes and buffers
-        rowsDir_ = rowsUpd_ = rowsRho_ = 0;
-        lanesDir_ = 0;
-        setupKindMaps();
-        // the sweeps take the same shape until reshapeSweeps
-        reshapeSweeps(lanes_, rowsPerBlock_);
     }
 
     int McgsSolver::minRowsPerBlock() const
@@ -851,7 +857,7 @@ namespace nsfem
             {
                 bmPre_ = flatMap(rowsPrecond_, nbPre_, 1024);
             }
-            if (regionDir_ && n_ > 0)
+            if (regionDir_ && n_ > 0 && !local())
             {
                 regionMap(bmDir_, nbDir_, dirTable_);
                 if (ownPrecondMap)
@@ -872,11 +878,343 @@ namespace nsfem
             nbDir_ = nbUpd_ = nbRho_ = nbPre_ = numBlocks_;
             color0BlocksRho_ = color0Blocks_;
         }
+        if (sliced())
+        {
+            setupSliceMaps();
+            maxBlocks = std::max(maxBlocks, nbDir_);
+        }
         // reduction scratch sized by the largest block count
         inner_.init(maxBlocks, numSystems_, opt_.numCh);
         if (opt_.precision == SolverPrecision::Mixed)
         {
             outer_.init(maxBlocks, numSystems_, opt_.numCh);
+        }
+    }
+
+    void McgsSolver::buildLocal(const std::vector<int> & rowStart, const std::vector<int> & rowSplit, const std::vector<int> & column,
+                                const std::vector<double> & values, const std::vector<double> & diag, const std::vector<double> & g,
+                                const std::vector<double> & gDiag)
+    {
+        const std::vector<int> perm = perm_.download(); // colour-major row -> original row
+        // systems one after another, each by locality rank (rank keeps a
+        // component's rows together, and systems share no entry)
+        std::vector<int> rank = localityRank(rowStart, column, n_);
+        std::vector<int> order(n_), systemOf(n_);
+        for (const RowChunk & ch : chunks_)
+        {
+            for (int r = ch.begin; r < ch.end; r++)
+            {
+                systemOf[r] = ch.system;
+            }
+        }
+        for (int i = 0; i < n_; i++)
+        {
+            order[rank[i]] = i;
+        }
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return systemOf[a] < systemOf[b]; });
+        loc_.chunks.clear();
+        for (int s = 0, at = 0; s < numSystems_; s++)
+        {
+            loc_.chunks.push_back(RowChunk{0, s, at, at + sysRows_[s]});
+            at += sysRows_[s];
+        }
+        // inside windows of the locality order: by entry count, then by the
+        // lower-colour part's, so that the 64 rows of a slice need little
+        // padding (P2 mass matrix of 2M rows: 21.2M entries sliced for 21.0M,
+        // the factor's halves 12.6M and 11.3M; windows of 256 rows pad
+        // the halves to 17M, windows of 4,096 spread a slice's gathers, 3 % slower)
+        for (const RowChunk & ch : loc_.chunks)
+        {
+            for (int w0 = ch.begin; w0 < ch.end; w0 += kSortWindow)
+            {
+                std::stable_sort(order.begin() + w0, order.begin() + std::min(ch.end, w0 + kSortWindow),
+                                 [&](int a, int b)
+                                 {
+                                     const int la = rowStart[a + 1] - rowStart[a], lb = rowStart[b + 1] - rowStart[b];
+                                     return la != lb ? la < lb : rowSplit[a] - rowStart[a] < rowSplit[b] - rowStart[b];
+                                 });
+            }
+        }
+        std::vector<int> pos(n_);
+        for (int i = 0; i < n_; i++)
+        {
+            pos[order[i]] = i;
+        }
+        std::vector<int> lperm(n_), liperm(n_), rs(n_ + 1, 0), split(n_), col(column.size());
+        std::vector<double> av(column.size()), gv(column.size()), ad(n_), gd(n_), inv(n_);
+        for (int i = 0; i < n_; i++)
+        {
+            const int o = order[i];
+            lperm[i] = perm[o];
+            liperm[perm[o]] = i;
+            rs[i + 1] = rs[i] + (rowStart[o + 1] - rowStart[o]);
+            split[i] = rs[i] + (rowSplit[o] - rowStart[o]);
+            ad[i] = diag[o];
+            inv[i] = 1.0 / diag[o];
+            gd[i] = gDiag[o];
+        }
+        std::vector<std::pair<int, int>> e;
+        for (int i = 0; i < n_; i++)
+        {
+            const int o = order[i];
+            auto part = [&](int from, int to, int at)
+            {
+                e.clear();
+                for (int j = from; j < to; j++)
+                {
+                    e.emplace_back(pos[column[j]], j);
+                }
+                std::sort(e.begin(), e.end());
+                for (const auto & [c, j] : e)
+                {
+                    col[at] = c;
+                    av[at] = values[j];
+                    gv[at] = g[j];
+                    at++;
+                }
+            };
+            part(rowStart[o], rowSplit[o], rs[i]);
+            part(rowSplit[o], rowStart[o + 1], split[i]);
+        }
+        if (col.empty())
+        {
+            col.push_back(0); // a diagonal matrix: keep valid pointers
+            av.push_back(0.0);
+            gv.push_back(0.0);
+        }
+        loc_.perm.upload(lperm);
+        loc_.iperm.upload(liperm);
+        if (opt_.precision == SolverPrecision::F32)
+        {
+            uploadMatrix(loc_.A32, rs, split, col, av, ad, inv);
+        }
+        else
+        {
+            uploadMatrix(loc_.A64, rs, split, col, av, ad, inv);
+        }
+        const bool p64 = opt_.precision == SolverPrecision::F64;
+        auto to32 = [](const std::vector<double> & v) { return std::vector<float>(v.begin(), v.end()); };
+        if (p64)
+        {
+            loc_.g64.upload(gv);
+            loc_.gDiag64.upload(gd);
+        }
+        else
+        {
+            loc_.g32.upload(to32(gv));
+            loc_.gDiag32.upload(to32(gd));
+        }
+        if (opt_.numCh > 2)
+        {
+            return;
+        }
+        // Slices of 64 rows of one system, entry k of all its rows side by
+        // side; a row's padding is 0 times its own element.
+        auto slice = [&](Slices & to, auto && range, const std::vector<double> & v, bool f64)
+        {
+            std::vector<int4> table;
+            std::vector<int> sc;
+            std::vector<double> sv;
+            loc_.systemSlice.assign(1, 0);
+            for (const RowChunk & ch : loc_.chunks)
+            {
+                for (int r0 = ch.begin; r0 < ch.end; r0 += 64)
+                {
+                    const int rows = std::min(64, ch.end - r0);
+                    int width = 0;
+                    for (int l = 0; l < rows; l++)
+                    {
+                        const auto [b, e] = range(r0 + l);
+                        width = std::max(width, e - b);
+                    }
+                    if (sc.size() + static_cast<size_t>(width + 1) * 64 > 0x7fffffffu)
+                    {
+                        throw std::invalid_argument("approximate inverse: the sliced system exceeds 32-bit indices");
+                    }
+                    const int at = static_cast<int>(sc.size());
+                    table.push_back(int4{r0, rows, at, width});
+                    sc.resize(at + static_cast<size_t>(width) * 64, r0);
+                    sv.resize(at + static_cast<size_t>(width) * 64, 0.0);
+                    for (int l = 0; l < rows; l++)
+                    {
+                        const auto [b, e] = range(r0 + l);
+                        for (int k = 0; k < width; k++)
+                        {
+                            const bool has = b + k < e;
+                            sc[at + 64 * k + l] = has ? col[b + k] : r0 + l;
+                            sv[at + 64 * k + l] = has ? v[b + k] : 0.0;
+                        }
+                    }
+                }
+                loc_.systemSlice.push_back(static_cast<int>(table.size()));
+            }
+            if (sc.empty())
+            {
+                sc.push_back(0);
+                sv.push_back(0.0);
+            }
+            to.slices.upload(table);
+            to.column.upload(sc);
+            if (f64)
+            {
+                to.values64.upload(sv);
+            }
+            else
+            {
+                to.values32.upload(to32(sv));
+            }
+        };
+        slice(loc_.a, [&](int r) { return std::pair<int, int>(rs[r], rs[r + 1]); }, av, opt_.precision != SolverPrecision::F32);
+        slice(loc_.lower, [&](int r) { return std::pair<int, int>(rs[r], split[r]); }, gv, p64);
+        slice(loc_.upper, [&](int r) { return std::pair<int, int>(split[r], rs[r + 1]); }, gv, p64);
+    }
+
+    void McgsSolver::setupSliceMaps()
+    {
+        // Each system's slices go to its share of kSliceGroups workgroups; every
+        // kernel of the iteration uses the same workgroups, so all partial
+        // sums share their slots.
+        const int total = loc_.systemSlice.back();
+        // Few slices: smaller workgroups reach more CUs (P2 mass matrix, two
+        // channels, us per iteration with 2 / 4 / 8 waves: 115 slices 16.1 /
+        // 16.8 / 18.8, 690 slices 18.8 / 17.8 / 19.1, 1,890 slices 30.5 / 26.1
+        // / 25.7, 7,550 slices 65.7 / 51.8 / 49.4).
+        loc_.waves = total > 1024 ? 8 : (total > 256 ? 4 : 2);
+        const int per = std::max(loc_.waves, (total + kSliceGroups - 1) / kSliceGroups); // slices per workgroup
+        std::vector<int> start(1, 0);
+        for (int s = 0; s < numSystems_; s++)
+        {
+            const int n = loc_.systemSlice[s + 1] - loc_.systemSlice[s];
+            start.push_back(start.back() + std::max(1, (n + per - 1) / per));
+        }
+        const int nb = start.back();
+        loc_.sysBlockStart.upload(start);
+        std::vector<int4> rows, slices;
+        for (int s = 0; s < numSystems_; s++)
+        {
+            const int k = start[s + 1] - start[s];
+            const int s0 = loc_.systemSlice[s], n = loc_.systemSlice[s + 1] - s0;
+            const RowChunk & ch = loc_.chunks[s];
+            for (int i = 0; i < k; i++)
+            {
+                const int a = static_cast<int>(static_cast<long>(n) * i / k), b = static_cast<int>(static_cast<long>(n) * (i + 1) / k);
+                slices.push_back(int4{s0 + a, s0 + b, s, start[s] + i});
+                rows.push_back(int4{ch.begin + 64 * a, std::min(ch.end, ch.begin + 64 * b), s, start[s] + i});
+            }
+        }
+        loc_.rowBlocks.upload(rows);
+        loc_.sliceBlocks.upload(slices);
+        loc_.rows = BlockMap{loc_.rowBlocks.get(), loc_.sysBlockStart.get(), nullptr, systemRows_.get(), numSystems_, nb, 0, 0, nullptr};
+        loc_.slices = loc_.rows;
+        loc_.slices.blocks = loc_.sliceBlocks.get();
+        // the reported rows per workgroup stay those of the lane-split maps
+        for (BlockMap * m : {&bmDir_, &bmUpd_, &bmPre_})
+        {
+            const int reported = m->rowsPerBlock;
+            *m = loc_.rows;
+            m->rowsPerBlock = reported;
+        }
+        nbDir_ = nbUpd_ = nbPre_ = nb;
+    }
+
+    template <typename F>
+    void McgsSolver::dispatchWaves(F && f) const
+    {
+        switch (loc_.waves)
+        {
+        case 2: f.template operator()<2>(); break;
+        case 4: f.template operator()<4>(); break;
+        default: f.template operator()<8>(); break;
+        }
+    }
+
+    template <typename T, typename P>
+    void McgsSolver::launchInit(hipStream_t s, const PcgOperands<T, P> & v, SolveState st, bool zeroGuess, const int * gate, double * totals)
+    {
+        const int nch = opt_.numCh;
+        if (sliced() && !zeroGuess)
+        {
+            const SlicedMatrix<T> A = loc_.a.view<T>();
+            dispatchWaves([&]<int W>()
+                      {
+                          auto go = [&]<int C>()
+                          { slicedInitKernel<T, P, W, C><<<nbDir_, 64 * W, 0, s>>>(A, v.A.diag, loc_.slices, st, v.b, v.x, v.r, v.rP); };
+                          nch == 1 ? go.template operator()<1>() : go.template operator()<2>();
+                      });
+        }
+        else
+        {
+            // r = b - A x is the direction kernel's product: its map and lanes
+            dispatchLC(directionLanes(), nch, [&]<int L, int C>()
+                       {
+                           pcgInitKernel<T, P, L, C><<<nbDir_, kBlock, 0, s>>>(v.A, bmDir_, st, v.b, v.x, v.r, v.rP, v.z, v.M.invDiag,
+                                                                              zColour0End(), zeroGuess ? 1 : 0);
+                       });
+        }
+        dispatchC(nch, [&]<int C>() { pcgInitFinalizeKernel<C><<<1, kFinBlock, 0, s>>>(bmDir_, st, gate, totals); });
+    }
+
+    template <typename T, typename P>
+    void McgsSolver::launchDirection(hipStream_t s, const PcgOperands<T, P> & v, SolveState st)
+    {
+        const int nch = opt_.numCh;
+        const int fz = fused() ? 1 : 0;
+        if (sliced())
+        {
+            const SlicedMatrix<T> A = loc_.a.view<T>();
+            dispatchWaves([&]<int W>()
+                      {
+                          auto go = [&]<int C>()
+                          { slicedDirectionKernel<T, P, W, C><<<nbDir_, 64 * W, 0, s>>>(A, v.A.diag, loc_.slices, st, v.z, v.p, v.q); };
+                          nch == 1 ? go.template operator()<1>() : go.template operator()<2>();
+                      });
+            return;
+        }
+        dispatchLC(directionLanes(), nch, [&]<int L, int C>()
+                   {
+                       pcgDirectionKernel<T, P, L, C><<<nbDir_, kBlock, 0, s>>>(v.A, bmDir_, st, v.z, v.p, v.q, fz, rhoParts(), nbUpd_);
+                   });
+    }
+
+    template <typename T, typename P>
+    void McgsSolver::launchApproximateInverse(hipStream_t s, const PcgOperands<T, P> & v, SolveState st)
+    {
+        const int nch = opt_.numCh;
+        if (sliced())
+        {
+            dispatchWaves([&]<int W>()
+                      {
+                          auto go = [&]<int C>()
+                          {
+                              slicedLowerKernel<P, W, C><<<nbPre_, 64 * W, 0, s>>>(loc_.lower.view<P>(), v.G.diag, loc_.slices, st, v.rP, v.t);
+                              slicedUpperKernel<P, T, W, C><<<nbPre_, 64 * W, 0, s>>>(loc_.upper.view<P>(), v.G.diag, loc_.slices, st, v.t,
+                                                                                     v.z, v.r);
+                          };
+                          nch == 1 ? go.template operator()<1>() : go.template operator()<2>();
+                      });
+            return;
+        }
+        dispatchLC(directionLanes(), nch, [&]<int L, int C>()
+                   {
+                       fsaiLowerKernel<P, L, C><<<nbPre_, kBlock, 0, s>>>(v.G, bmPre_, st, v.rP, v.t);
+                       fsaiUpperKernel<P, T, L, C><<<nbPre_, kBlock, 0, s>>>(v.G, bmPre_, st, v.t, v.z, v.r);
+                   });
+    }
+
+    void McgsSolver::setMixedRestart(bool on)
+    {
+        if (opt_.restart == on)
+        {
+            return;
+        }
+        NSFEM_HIP(hipStreamSynchronize(stream_));
+        opt_.restart = on;
+        if (precond_ == 1)
+        {
+            // refinement's inner solves run in colour order
+            setupMainMap();
+            setupKindMaps();
+            destroyGraphs();
         }
     }
 
@@ -1146,21 +1484,24 @@ namespace nsfem
     template <>
     PcgOperands<double, double> McgsSolver::operands<double, double>()
     {
-        return {A64_.view(n_), A64_.view(n_), b64_.get(), x64_.get(), r64_.get(), r64_.get(), z64_.get(), p64_.get(), q64_.get(),
+        const McgsMatrix<double> A = local() ? loc_.A64.view(n_) : A64_.view(n_);
+        return {A, A, b64_.get(), x64_.get(), r64_.get(), r64_.get(), z64_.get(), p64_.get(), q64_.get(),
                 fsaiView<double>(), reinterpret_cast<double *>(fsaiT_.get())};
     }
 
     template <>
     PcgOperands<float, float> McgsSolver::operands<float, float>()
     {
-        return {A32_.view(n_), A32_.view(n_), b32_.get(), x32_.get(), r32_.get(), r32_.get(), z32_.get(), p32_.get(), q32_.get(),
+        const McgsMatrix<float> A = local() && opt_.precision == SolverPrecision::F32 ? loc_.A32.view(n_) : A32_.view(n_);
+        return {A, A, b32_.get(), x32_.get(), r32_.get(), r32_.get(), z32_.get(), p32_.get(), q32_.get(),
                 fsaiView<float>(), reinterpret_cast<float *>(fsaiT_.get())};
     }
 
     template <>
     PcgOperands<double, float> McgsSolver::operands<double, float>()
     {
-        return {A64_.view(n_), A32_.view(n_), b64_.get(), x64_.get(), r64_.get(), r32_.get(), z32_.get(), p64_.get(), q64_.get(),
+        // (in locality order the preconditioner is G alone: M is not used)
+        return {local() ? loc_.A64.view(n_) : A64_.view(n_), A32_.view(n_), b64_.get(), x64_.get(), r64_.get(), r32_.get(), z32_.get(), p64_.get(), q64_.get(),
                 fsaiView<float>(), reinterpret_cast<float *>(fsaiT_.get())};
     }
 
@@ -1278,14 +1619,11 @@ namespace nsfem
         const int nch = opt_.numCh;
         double * totals = inner_.totals.get();
         const int fz = fused() ? 1 : 0;
-        dispatchLC(directionLanes(), nch, [&]<int L, int C>()
-                   {
-                       pcgDirectionKernel<T, P, L, C><<<nbDir_, kBlock, 0, s>>>(v.A, bmDir_, st, v.z, v.p, v.q, fz, rhoParts(), nbUpd_);
-                       if (!fz)
-                       {
-                           pcgDirectionFinalizeKernel<C><<<1, kFinBlock, 0, s>>>(bm_, st, totals);
-                       }
-                   });
+        launchDirection<T, P>(s, v, st);
+        if (!fz)
+        {
+            dispatchC(nch, [&]<int C>() { pcgDirectionFinalizeKernel<C><<<1, kFinBlock, 0, s>>>(bm_, st, totals); });
+        }
         if (mergedUpdate())
         {
             launchUpdateSweep<T, P>(s, v, st);
@@ -1311,21 +1649,11 @@ namespace nsfem
             launchRho<T, P>(s, v, st, totals, withUpdate);
             return;
         }
-        // on a region-major map (the workgroups of one XCD take the same
-        // stretch of every colour and gather from about an eighth of the
-        // vector): the direction kernel's, or one with rows of its own
-        // (rowsPreconditioner); the next direction kernel reads nbPre_ rho
-        // partials
-        const bool fin = !fused();
-        dispatchLC(directionLanes(), opt_.numCh, [&]<int L, int C>()
-                   {
-                       fsaiLowerKernel<P, L, C><<<nbPre_, kBlock, 0, s>>>(v.G, bmPre_, st, v.rP, v.t);
-                       fsaiUpperKernel<P, T, L, C><<<nbPre_, kBlock, 0, s>>>(v.G, bmPre_, st, v.t, v.z, v.r);
-                       if (fin)
-                       {
-                           pcgRhoFinalizeKernel<C><<<1, kFinBlock, 0, s>>>(bm_, st, totals, withUpdate ? 1 : 0);
-                       }
-                   });
+        launchApproximateInverse<T, P>(s, v, st);
+        if (!fused())
+        {
+            dispatchC(opt_.numCh, [&]<int C>() { pcgRhoFinalizeKernel<C><<<1, kFinBlock, 0, s>>>(bm_, st, totals, withUpdate ? 1 : 0); });
+        }
     }
 
     template <typename P>
@@ -1334,9 +1662,9 @@ namespace nsfem
         // the structure of the preconditioner's matrix, the factor's values
         if constexpr (std::is_same_v<P, double>)
         {
-            McgsMatrix<double> G = A64_.view(n_);
-            G.values = fsai64_.get();
-            G.diag = fsaiDiag64_.get();
+            McgsMatrix<double> G = local() ? loc_.A64.view(n_) : A64_.view(n_);
+            G.values = local() ? loc_.g64.get() : fsai64_.get();
+            G.diag = local() ? loc_.gDiag64.get() : fsaiDiag64_.get();
             G.invDiag = nullptr;
             return G;
         }
@@ -1345,6 +1673,15 @@ namespace nsfem
             McgsMatrix<float> G = A32_.view(n_);
             G.values = fsai32_.get();
             G.diag = fsaiDiag32_.get();
+            if (local())
+            {
+                const bool f32 = opt_.precision == SolverPrecision::F32;
+                G.rowStart = f32 ? loc_.A32.rowStart.get() : loc_.A64.rowStart.get();
+                G.rowSplit = f32 ? loc_.A32.rowSplit.get() : loc_.A64.rowSplit.get();
+                G.column = f32 ? loc_.A32.column.get() : loc_.A64.column.get();
+                G.values = loc_.g32.get();
+                G.diag = loc_.gDiag32.get();
+            }
             G.invDiag = nullptr;
             return G;
         }
@@ -1388,7 +1725,10 @@ namespace nsfem
                     diag.assign(d32.begin(), d32.end());
                 }
                 std::vector<double> g, gd;
+                column.resize(rowStart[n_]); // (a diagonal matrix's arrays hold one entry)
+                values.resize(rowStart[n_]);
                 buildFsai(n_, rowStart, rowSplit, column, values, diag, g, gd);
+                buildLocal(rowStart, rowSplit, column, values, diag, g, gd);
                 if (column.empty())
                 {
                     g.assign(1, 0.0); // a diagonal matrix: keep a valid pointer
@@ -1411,7 +1751,12 @@ namespace nsfem
             }
         }
         NSFEM_HIP(hipStreamSynchronize(stream_));
-        precond_ = kind;
+        if (precond_ != kind)
+        {
+            precond_ = kind;
+            setupMainMap();
+            setupKindMaps();
+        }
         destroyGraphs();
     }
 
@@ -1422,13 +1767,7 @@ namespace nsfem
         const int nch = opt_.numCh;
         double * totals = inner_.totals.get();
         fillInt(4, 0, st.flags, s);
-        // r = b - A x is the direction kernel's product: its map and lanes
-        dispatchLC(directionLanes(), nch, [&]<int L, int C>()
-                   {
-                       pcgInitKernel<T, P, L, C><<<nbDir_, kBlock, 0, s>>>(v.A, bmDir_, st, v.b, v.x, v.r, v.rP, v.z, v.M.invDiag,
-                                                                          zColour0End(), zeroGuess ? 1 : 0);
-                       pcgInitFinalizeKernel<C><<<1, kFinBlock, 0, s>>>(bmDir_, st, gate, totals);
-                   });
+        launchInit<T, P>(s, v, st, zeroGuess, gate, totals);
         launchPrecond<T, P>(s, v, st, totals, false);
         NSFEM_HIP(hipGetLastError());
         return iterate<T, P>(s, v, st, maxIters, sync, usePrediction);
@@ -1907,10 +2246,23 @@ namespace nsfem
     void McgsSolver::permuteRows(int dt, const void * src, void * dst, bool inverse, hipStream_t s)
     {
         const int nch = opt_.numCh;
-        if (nch > 2 || n_ <= 0 || !(inverse || bmDir_.rowTable))
+        const int * perm = local() ? loc_.perm.get() : perm_.get();
+        const int * iperm = local() ? loc_.iperm.get() : iperm_.get();
+        if (nch > 2 || n_ <= 0 || !(inverse || local() || bmDir_.rowTable))
         {
-            permute(dt, dt, n_, nch, perm_.get(), src, dst, inverse, s);
+            permute(dt, dt, n_, nch, perm, src, dst, inverse, s);
             return;
+        }
+        // into locality order: flat workgroups (neighbouring rows come from
+        // neighbouring places already)
+        BlockMap map = bmDir_;
+        int blocks = nbDir_;
+        if (local())
+        {
+            map.flatRows = n_;
+            map.rowsPerBlock = 4 * kBlock;
+            map.rowTable = nullptr;
+            blocks = (n_ + map.rowsPerBlock - 1) / map.rowsPerBlock;
         }
         const int inv = inverse ? 1 : 0;
         auto go = [&]<typename T>()
@@ -1922,20 +2274,20 @@ namespace nsfem
                 const int g = (n_ + kBlock - 1) / kBlock;
                 if (nch == 1)
                 {
-                    unpermuteGatherKernel<T, T, 1><<<g, kBlock, 0, s>>>(n_, iperm_.get(), sp, dp);
+                    unpermuteGatherKernel<T, T, 1><<<g, kBlock, 0, s>>>(n_, iperm, sp, dp);
                 }
                 else
                 {
-                    unpermuteGatherKernel<T, T, 2><<<g, kBlock, 0, s>>>(n_, iperm_.get(), sp, dp);
+                    unpermuteGatherKernel<T, T, 2><<<g, kBlock, 0, s>>>(n_, iperm, sp, dp);
                 }
             }
             else if (nch == 1)
             {
-                permuteMappedKernel<T, T, 1><<<nbDir_, kBlock, 0, s>>>(bmDir_, n_, perm_.get(), sp, dp, inv);
+                permuteMappedKernel<T, T, 1><<<blocks, kBlock, 0, s>>>(map, n_, perm, sp, dp, inv);
             }
             else
             {
-                permuteMappedKernel<T, T, 2><<<nbDir_, kBlock, 0, s>>>(bmDir_, n_, perm_.get(), sp, dp, inv);
+                permuteMappedKernel<T, T, 2><<<blocks, kBlock, 0, s>>>(map, n_, perm, sp, dp, inv);
             }
         };
         if (dt == F64)
@@ -1970,12 +2322,7 @@ namespace nsfem
         const int nch = opt_.numCh;
         double * totals = inner_.totals.get();
         fillInt(4, 0, st.flags, s);
-        dispatchLC(directionLanes(), nch, [&]<int L, int C>()
-                   {
-                       pcgInitKernel<T, P, L, C><<<nbDir_, kBlock, 0, s>>>(v.A, bmDir_, st, v.b, v.x, v.r, v.rP, v.z, v.M.invDiag,
-                                                                          zColour0End(), zeroGuess ? 1 : 0);
-                       pcgInitFinalizeKernel<C><<<1, kFinBlock, 0, s>>>(bmDir_, st, nullptr, totals);
-                   });
+        launchInit<T, P>(s, v, st, zeroGuess, nullptr, totals);
         launchPrecond<T, P>(s, v, st, totals, false);
         for (int i = 0; i < budget; i++)
         {
@@ -2202,14 +2549,7 @@ namespace nsfem
             {
                 // matrix and diagonal, z gathered once, p and q read and written
                 bytes = nnzOff * (tsT + 4.0) + (n + 1) * 4.0 + n * tsT + nch * (n * tsP + 4.0 * n * tsT);
-                launch = [=, this]()
-                {
-                    dispatchLC(directionLanes(), nch, [&]<int L, int C>()
-                               {
-                                   pcgDirectionKernel<T, P, L, C><<<nbDir_, kBlock, 0, s>>>(v.A, bmDir_, st, v.z, v.p, v.q, fz, rhoParts(),
-                                                                                            nbUpd_);
-                               });
-                };
+                launch = [=, this]() { launchDirection<T, P>(s, v, st); };
             }
             else if (which == "sweep")
             {
@@ -2278,14 +2618,7 @@ namespace nsfem
                 }
                 launches = 2;
                 bytes = (full * (tsP + 4.0) + 2.0 * ((n + 1) * 4.0 + n * 4.0 + n * tsP) + nch * n * (4.0 * tsP + tsT)) / 2.0;
-                launch = [=, this]()
-                {
-                    dispatchLC(directionLanes(), nch, [&]<int L, int C>()
-                               {
-                                   fsaiLowerKernel<P, L, C><<<nbPre_, kBlock, 0, s>>>(v.G, bmPre_, st, v.rP, v.t);
-                                   fsaiUpperKernel<P, T, L, C><<<nbPre_, kBlock, 0, s>>>(v.G, bmPre_, st, v.t, v.z, v.r);
-                               });
-                };
+                launch = [=, this]() { launchApproximateInverse<T, P>(s, v, st); };
             }
             else if (which == "update")
             {
@@ -2310,7 +2643,7 @@ namespace nsfem
                         dispatchC(nch, [&]<int C>()
                                   {
                                       pcgUpdateKernel<T, P, C><<<nbUpd_, kBlock, 0, s>>>(n_, bmUpd_, st, v.p, v.q, v.x, v.r, v.rP,
-                                                                                        v.z, v.M.invDiag, color0End_, fz, nbDir_);
+                                                                                        v.z, v.M.invDiag, zColour0End(), fz, nbDir_);
                                   });
                     };
                 }

@@ -30,6 +30,7 @@
 #include "bcg_kernels.hpp"
 #include "kernels.hpp"
 #include "ops.hpp"
+#include "sliced_kernels.hpp"
 
 namespace nsfem
 {
@@ -180,7 +181,7 @@ namespace nsfem
         void setTarget(double t) { opt_.target = t; }
         void setMseCheckInterval(int k);
         void setInnerTol(double t) { opt_.innerTol = t; }
-        void setMixedRestart(bool on) { opt_.restart = on; }
+        void setMixedRestart(bool on);
         void setProjectMean(bool on) { opt_.projectMean = on; }
         // block PCG: relative pivot threshold of the rho = Z^T R
         // factorisation (0: 1e-13 with an FP64 preconditioner, 1e-10 with FP32)
@@ -201,8 +202,9 @@ namespace nsfem
         // larger blocks pay there.  reshape resets them.
         void setKindRows(int direction, int update, int rho);
         // Rows per workgroup of the approximate inverse's two launches
-        // (preconditioner = 1; fused reductions on one system): 0 (default)
-        // shares the direction kernel's map, else a positive multiple of 256.
+        // (preconditioner = 1; fused reductions on one system, wide tiles): 0
+        // (default) shares the direction kernel's map, else a positive multiple
+        // of 256; no effect on sliced rows (1 and 2 channels).
         void setPreconditionerRows(int rows);
         int preconditionerRows() const { return rowsPrecond_; }
         int kindRows(int kind) const; // 0 direction, 1 update, 2 rho
@@ -317,6 +319,24 @@ namespace nsfem
         int rhoParts() const { return precond_ == 0 ? nbRho_ : nbPre_; }
         template <typename P>
         McgsMatrix<P> fsaiView() const;
+        // The approximate inverse needs no colour order: its solves run on a
+        // copy of the system with the rows of every system in locality order.
+        bool local() const { return precond_ == 1 && !opt_.restart; }
+        // ... and, with fused reductions on one or two channels, its products
+        // on slices of 64 rows (sliced_kernels.hpp)
+        bool sliced() const { return local() && fused() && opt_.numCh <= 2; }
+        void buildLocal(const std::vector<int> & rowStart, const std::vector<int> & rowSplit, const std::vector<int> & column,
+                        const std::vector<double> & values, const std::vector<double> & diag, const std::vector<double> & g,
+                        const std::vector<double> & gDiag);
+        // f<W>() for the waves per workgroup of the sliced kernels
+        template <typename F>
+        void dispatchWaves(F && f) const;
+        template <typename T, typename P>
+        void launchInit(hipStream_t s, const PcgOperands<T, P> & v, SolveState st, bool zeroGuess, const int * gate, double * totals);
+        template <typename T, typename P>
+        void launchDirection(hipStream_t s, const PcgOperands<T, P> & v, SolveState st);
+        template <typename T, typename P>
+        void launchApproximateInverse(hipStream_t s, const PcgOperands<T, P> & v, SolveState st);
         void runMixedRestart(hipStream_t s);
         template <typename P>
         void runBlockPcg(hipStream_t s, const McgsMatrix<P> & M, P * rP, P * z, bool zeroGuess);
@@ -383,7 +403,11 @@ namespace nsfem
         DeviceArray<int4> sweepBlocks_;
         BlockMap sweepBm_{};
         std::pair<int, int> resolveShape(int lanes, int rowsPerBlock, bool sweeps) const;
-        void buildBlocks(int rpb, std::vector<int4> & blocks, std::vector<int> & blockSystem, std::vector<int> & colorStart) const;
+        void buildBlocks(const std::vector<RowChunk> & chunks, int rpb, std::vector<int4> & blocks, std::vector<int> & blockSystem,
+                         std::vector<int> & colorStart) const;
+        // bm_ from the main shape, over the colour-major rows or (local()) the
+        // systems in locality order
+        void setupMainMap();
         void destroyGraphs();
 
         DeviceArray<int> perm_;
@@ -424,6 +448,44 @@ namespace nsfem
         hipStream_t stream_;
 
         int precond_ = 0;
+        // The system in locality order for the approximate inverse, built
+        // when it is first chosen: A in its own precision, the factor in the
+        // preconditioner's, one row structure (lower-colour entries first).
+        struct Slices // one product's entries, sliced
+        {
+            DeviceArray<int4> slices;
+            DeviceArray<int> column;
+            DeviceArray<double> values64;
+            DeviceArray<float> values32;
+            template <typename T>
+            SlicedMatrix<T> view() const
+            {
+                if constexpr (std::is_same_v<T, double>)
+                {
+                    return {slices.get(), column.get(), values64.get()};
+                }
+                else
+                {
+                    return {slices.get(), column.get(), values32.get()};
+                }
+            }
+        };
+        struct Local
+        {
+            DeviceArray<int> perm, iperm;
+            DeviceMcgs<double> A64;
+            DeviceMcgs<float> A32;
+            DeviceArray<double> g64, gDiag64;
+            DeviceArray<float> g32, gDiag32;
+            std::vector<RowChunk> chunks;   // one per system
+            std::vector<int> systemSlice;   // numSystems + 1
+            int waves = 8;                  // per workgroup of the sliced kernels
+            Slices a, lower, upper;
+            DeviceArray<int4> rowBlocks, sliceBlocks;
+            DeviceArray<int> sysBlockStart;
+            BlockMap rows{}, slices{}; // the same workgroups as ranges of rows and of slices
+        } loc_;
+        void setupSliceMaps();
         DeviceArray<double> fsai64_, fsaiDiag64_;
         DeviceArray<float> fsai32_, fsaiDiag32_;
         DeviceArray<char> fsaiT_;

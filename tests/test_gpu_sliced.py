@@ -1,0 +1,104 @@
+"""PCG with the approximate inverse on sliced rows in locality order against
+the general kernels (two finalize launches per iteration, which walk the same
+rows in CSR form): edges of the slices, empty and long rows, several systems."""
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+import scipy.sparse.linalg as spla
+
+pytestmark = pytest.mark.gpu
+
+
+def _spd(n, seed, kind):
+    """Symmetric, strictly diagonally dominant (so SPD): condition below 20."""
+    rng = np.random.default_rng(seed)
+    if kind == "diagonal":
+        return sp.diags(rng.uniform(1, 2, n)).tocsr()
+    a = sp.random(n, n, min(1.0, 6.0 / n), random_state=rng, format="lil" if kind == "long" else "csr")
+    if kind == "long":  # rows of very different length, some empty off the diagonal
+        for r in range(0, n, 97):
+            a[r, rng.integers(0, n, min(n, 150))] = 0.3
+        a[n // 2:, :] = 0
+    a = a.tocsr()
+    a = a + a.T
+    a.setdiag(0)
+    a.eliminate_zeros()
+    return (a + sp.diags(np.asarray(abs(a).sum(axis=1)).ravel() * 1.2 + 1)).tocsr()
+
+
+def _run(name, nch, mats, b, x0, fused, dtype, target):
+    from nsfem_amd import cu
+    make = cu.createSolver if len(mats) == 1 else cu.createBatchSolver
+    s = make(name, nch, mats[0] if len(mats) == 1 else mats, 400, target, 1, dtype=dtype)
+    s.setOption("preconditioner", 1)
+    s.setOption("fusedReductions", fused)
+    s.getRhs().upload(b)
+    s.getSol().upload(x0)
+    s.solve()
+    return s, s.getSol().download().astype(np.float64)
+
+
+# 64 rows are a slice; 2, 4 and 8 waves a workgroup up to 256, 1,024 and more
+# slices; a window of 1,024 rows is sorted together
+@pytest.mark.parametrize("sizes", [[1], [63], [64], [65], [1023], [1025], [257 * 64 + 1], [1025 * 64 + 5], [40, 1, 700, 64, 130]])
+@pytest.mark.parametrize("name,nch,dtype", [("pcg", 1, np.float64), ("pcg", 2, np.float64), ("pcg_mixed", 2, np.float64),
+                                            ("pcg_mixed", 1, np.float64), ("pcg", 2, np.float32)])
+@pytest.mark.parametrize("kind", ["sparse", "long", "diagonal"])
+def test_sliced_solves_equal_the_general_kernels(sizes, name, nch, dtype, kind):
+    if kind != "sparse" and max(sizes) > 20_000:
+        pytest.skip("the long-row pattern is built densely")
+    mats = [_spd(n, 100 + n, kind) for n in sizes]
+    n = sum(sizes)
+    rng = np.random.default_rng(7)
+    b = rng.uniform(-1, 1, nch * n).astype(dtype)
+    x0 = rng.uniform(-1, 1, nch * n).astype(dtype)
+    target = 1e-12 if dtype == np.float64 else 1e-5
+    s, x = _run(name, nch, mats, b, x0, 1, dtype, target)
+    g, xg = _run(name, nch, mats, b, x0, 0, dtype, target)
+    # each solution is within cond * target of the exact one (cond < 20)
+    bound = 2 * 20 * target
+    assert np.linalg.norm(x - xg) <= bound * np.linalg.norm(xg)
+    assert abs(s.getLastIterations() - g.getLastIterations()) <= 1
+    # the true residual; in FP32 it drifts from the recursive one by a few roundings
+    slack = 1.01 * target + (0 if dtype == np.float64 else 16 * np.finfo(np.float32).eps)
+    start = 0
+    for m in mats:
+        rows = slice(start, start + m.shape[0])
+        start += m.shape[0]
+        for c in range(nch):
+            bc, xc = b[c * n:(c + 1) * n].astype(np.float64)[rows], x[c * n:(c + 1) * n][rows]
+            assert np.linalg.norm(bc - m @ xc) <= slack * np.linalg.norm(bc), (m.shape, c)
+
+
+def test_non_finite_right_hand_side_is_reported():
+    from nsfem_amd import cu
+    m = _spd(500, 3, "sparse")
+    s = cu.createSolver("pcg", 2, m, 50, 1e-10, 1)
+    s.setOption("preconditioner", 1)
+    b = np.ones(1000)
+    b[77] = np.nan
+    s.getRhs().upload(b)
+    s.getSol().memsetZero()
+    s.solve()
+    assert not np.isfinite(s.getLastMse(0))
+
+
+def test_preconditioner_switched_off_again_and_refinement_keep_working():
+    """The colour-major rows serve the GS sweeps and the refinement path; the
+    locality order only the approximate inverse."""
+    from nsfem_amd import cu
+    m = _spd(3000, 5, "sparse")
+    rng = np.random.default_rng(9)
+    b = rng.uniform(-1, 1, 3000)
+    ref = spla.spsolve(m.tocsc(), b)
+    s = cu.createSolver("pcg_mixed", 1, m, 400, 1e-11, 1)
+    for precond, restart in ((0, 0), (1, 0), (0, 0), (1, 0), (1, 1), (1, 0)):
+        s.setOption("mixedRestart", 0)
+        s.setOption("preconditioner", precond)
+        s.setOption("mixedRestart", restart)
+        s.getRhs().upload(b)
+        s.getSol().memsetZero()
+        s.solve()
+        x = s.getSol().download()
+        assert np.linalg.norm(x - ref) <= 20 * 1e-11 * np.linalg.norm(ref), (precond, restart)
