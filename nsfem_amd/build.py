@@ -13,7 +13,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libnsfem_hip.so")
 
-HIP_SOURCES = ["ops.hip", "solver.hip", "amg_pcg.hip", "chorin.hip", "capi.hip", "assembly.hip"]
+HIP_SOURCES = ["ops.hip", "solver.hip", "amg_pcg.hip", "dense_inverse.hip", "chorin.hip", "capi.hip", "assembly.hip"]
 # The GPU assembly evaluates the element integrals the host assembly shares
 # with it; without FP contraction both run the same IEEE operations.
 HIP_EXTRA_FLAGS = {"assembly.hip": ["-ffp-contract=off"]}

@@ -6,24 +6,67 @@
 #include <stdexcept>
 #include <type_traits>
 
+#include "dense_inverse.hpp"
 #include "ops.hpp"
 
 namespace nsfem
 {
     namespace
     {
-        struct AmgState
+        // Four channels or more: one lane per channel, E = L / NCH groups of
+        // NCH lanes on a row (lane g * NCH + c: channel c, every E-th entry
+        // from the g-th), so that a gathered column is NCH contiguous values
+        // and a short row is one round of loads.
+        template <int NCH>
+        constexpr bool kChannelLanes = NCH >= 4;
+
+        // Threads of the kernels that leave partial sums: many channels do many
+        // channels' work per row, and larger workgroups fill the chip without
+        // more partial sums (100k rows x 16, 395 workgroups: direction 40 -> 28 us).
+        template <int NCH>
+        constexpr int kCgBlock = kChannelLanes<NCH> ? 1024 : kBlock;
+
+        template <typename T, int L, int NCH, typename V>
+        __device__ __forceinline__ T rowDotChannels(const McgsMatrix<T> & A, int j0, int j1, const V * __restrict__ v)
         {
-            double * scal; // per channel, blocks of NCH: rho, rho of the iteration before, |b|^2, |r|^2
-            int * ints;    // stop (0 running, 1 converged, 2 non-finite or breakdown), iterations, zero right-hand sides
-            int * active;  // per channel
-            double * partPq;
-            double * partRr;
-            double * partRho;
-            double * partBb;
-            int parts;
-            double tol2;
-        };
+            constexpr int E = L / NCH, U = 4;
+            const int lane = static_cast<int>(threadIdx.x) % L;
+            const int c = lane % NCH, g = lane / NCH;
+            T acc = T(0);
+            for (int j = j0 + g; j < j1; j += E * U)
+            {
+                // past the row's end: the step's first entry again, its term dropped
+                T a[U];
+                int col[U];
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                {
+                    const int js = j + u * E < j1 ? j + u * E : j;
+                    a[u] = A.values[js];
+                    col[u] = A.column[js];
+                }
+                V x[U];
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                {
+                    x[u] = v[static_cast<long>(col[u]) * NCH + c];
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                {
+                    if (j + u * E < j1)
+                    {
+                        acc = fmaT(a[u], static_cast<T>(x[u]), acc);
+                    }
+                }
+            }
+#pragma unroll
+            for (int off = NCH; off < L; off <<= 1)
+            {
+                acc += __shfl_xor(acc, off, 64);
+            }
+            return acc;
+        }
 
         // ---------------- V-cycle (channels interleaved per row) ----------------
 
@@ -36,40 +79,67 @@ namespace nsfem
         __global__ void __launch_bounds__(kBlock) amgSweepKernel(McgsMatrix<T> A, int rowBegin, int rowEnd, const T * __restrict__ b,
                                                                  T * __restrict__ x, int lowerOnly, const int * __restrict__ stop)
         {
-            // The stop flag, the row bounds and the row's own operands load
-            // together, with no condition around a load (one would end in a
-            // wait for every load in flight): lanes past the colour read its
-            // first row and take no entries.
-            const int t = blockIdx.x * kBlock + threadIdx.x;
-            const int row = rowBegin + t / L;
-            const int lane = t % L;
-            const bool valid = row < rowEnd;
-            const int rs = valid ? row : rowBegin;
-            const int stopped = *stop;
-            const int * end = lowerOnly ? A.rowSplit : A.rowStart + 1;
-            const int j0 = A.rowStart[rs];
-            const int j1 = end[rs];
-            const T d = A.invDiag[rs];
-            T bi[NCH];
-#pragma unroll
-            for (int c = 0; c < NCH; c++)
+            if constexpr (kChannelLanes<NCH>)
             {
-                bi[c] = b[static_cast<long>(rs) * NCH + c];
-            }
-            // (j1 < j0 never holds; testing it keeps the loads ahead of the
-            // branch, where the compiler would otherwise sink them)
-            if (stopped | (j1 < j0))
-            {
+                const int t = blockIdx.x * kBlock + threadIdx.x;
+                const int row = rowBegin + t / L;
+                const bool valid = row < rowEnd;
+                const int rs = valid ? row : rowBegin;
+                const int stopped = *stop;
+                const int * end = lowerOnly ? A.rowSplit : A.rowStart + 1;
+                const int j0 = A.rowStart[rs];
+                const int j1 = end[rs];
+                const T d = A.invDiag[rs];
+                const long i = static_cast<long>(rs) * NCH + t % NCH;
+                const T bi = b[i];
+                if (stopped | (j1 < j0))
+                {
+                    return;
+                }
+                const T s = rowDotChannels<T, L, NCH>(A, j0, valid ? j1 : j0, x);
+                if (valid && t % L < NCH)
+                {
+                    x[i] = (bi - s) * d;
+                }
                 return;
             }
-            T s[NCH];
-            rowDot<T, L, NCH>(A, j0, valid ? j1 : j0, x, s);
-            if (valid && lane == 0)
+            else
             {
+                // The stop flag, the row bounds and the row's own operands load
+                // together, with no condition around a load (one would end in a
+                // wait for every load in flight): lanes past the colour read its
+                // first row and take no entries.
+                const int t = blockIdx.x * kBlock + threadIdx.x;
+                const int row = rowBegin + t / L;
+                const int lane = t % L;
+                const bool valid = row < rowEnd;
+                const int rs = valid ? row : rowBegin;
+                const int stopped = *stop;
+                const int * end = lowerOnly ? A.rowSplit : A.rowStart + 1;
+                const int j0 = A.rowStart[rs];
+                const int j1 = end[rs];
+                const T d = A.invDiag[rs];
+                T bi[NCH];
 #pragma unroll
                 for (int c = 0; c < NCH; c++)
                 {
-                    x[static_cast<long>(row) * NCH + c] = (bi[c] - s[c]) * d;
+                    bi[c] = b[static_cast<long>(rs) * NCH + c];
+                }
+                // (j1 < j0 never holds; testing it keeps the loads ahead of the
+                // branch, where the compiler would otherwise sink them)
+                if (stopped | (j1 < j0))
+                {
+                    return;
+                }
+                T s[NCH];
+                rowDot<T, L, NCH>(A, j0, valid ? j1 : j0, x, s);
+                if (valid && lane == 0)
+                {
+#pragma unroll
+                    for (int c = 0; c < NCH; c++)
+                    {
+                        x[static_cast<long>(row) * NCH + c] = (bi[c] - s[c]) * d;
+                    }
                 }
             }
         }
@@ -79,37 +149,63 @@ namespace nsfem
         __global__ void __launch_bounds__(kBlock) amgResidualKernel(McgsMatrix<T> A, const T * __restrict__ b, const T * __restrict__ x,
                                                                     T * __restrict__ r, const int * __restrict__ stop)
         {
-            const int t = blockIdx.x * kBlock + threadIdx.x;
-            const int row = t / L;
-            const int lane = t % L;
-            const bool valid = row < A.n;
-            const int rs = valid ? row : 0;
-            const int stopped = *stop;
-            const int j0 = A.rowStart[rs];
-            const int j1 = A.rowStart[rs + 1];
-            const T d = A.diag[rs];
-            T bi[NCH], xi[NCH];
-#pragma unroll
-            for (int c = 0; c < NCH; c++)
+            if constexpr (kChannelLanes<NCH>)
             {
-                const long i = static_cast<long>(rs) * NCH + c;
-                bi[c] = b[i];
-                xi[c] = x[i];
-            }
-            // (j1 < j0 never holds; testing it keeps the loads ahead of the
-            // branch, where the compiler would otherwise sink them)
-            if (stopped | (j1 < j0))
-            {
+                const int t = blockIdx.x * kBlock + threadIdx.x;
+                const int row = t / L;
+                const bool valid = row < A.n;
+                const int rs = valid ? row : 0;
+                const int stopped = *stop;
+                const int j0 = A.rowStart[rs];
+                const int j1 = A.rowStart[rs + 1];
+                const T d = A.diag[rs];
+                const long i = static_cast<long>(rs) * NCH + t % NCH;
+                const T bi = b[i], xi = x[i];
+                if (stopped | (j1 < j0))
+                {
+                    return;
+                }
+                const T s = rowDotChannels<T, L, NCH>(A, j0, valid ? j1 : j0, x);
+                if (valid && t % L < NCH)
+                {
+                    r[i] = bi - fmaT(d, xi, s);
+                }
                 return;
             }
-            T s[NCH];
-            rowDot<T, L, NCH>(A, j0, valid ? j1 : j0, x, s);
-            if (valid && lane == 0)
+            else
             {
+                const int t = blockIdx.x * kBlock + threadIdx.x;
+                const int row = t / L;
+                const int lane = t % L;
+                const bool valid = row < A.n;
+                const int rs = valid ? row : 0;
+                const int stopped = *stop;
+                const int j0 = A.rowStart[rs];
+                const int j1 = A.rowStart[rs + 1];
+                const T d = A.diag[rs];
+                T bi[NCH], xi[NCH];
 #pragma unroll
                 for (int c = 0; c < NCH; c++)
                 {
-                    r[static_cast<long>(row) * NCH + c] = bi[c] - fmaT(d, xi[c], s[c]);
+                    const long i = static_cast<long>(rs) * NCH + c;
+                    bi[c] = b[i];
+                    xi[c] = x[i];
+                }
+                // (j1 < j0 never holds; testing it keeps the loads ahead of the
+                // branch, where the compiler would otherwise sink them)
+                if (stopped | (j1 < j0))
+                {
+                    return;
+                }
+                T s[NCH];
+                rowDot<T, L, NCH>(A, j0, valid ? j1 : j0, x, s);
+                if (valid && lane == 0)
+                {
+#pragma unroll
+                    for (int c = 0; c < NCH; c++)
+                    {
+                        r[static_cast<long>(row) * NCH + c] = bi[c] - fmaT(d, xi[c], s[c]);
+                    }
                 }
             }
         }
@@ -125,42 +221,73 @@ namespace nsfem
                                                                 int accumulate, const int * __restrict__ stop, const T * __restrict__ initInv,
                                                                 T * __restrict__ xInit, T initScale)
         {
-            const int t = blockIdx.x * kBlock + threadIdx.x;
-            const int row = t / L;
-            const int lane = t % L;
-            const bool valid = row < rows;
-            const int rs = valid ? row : 0;
-            const int stopped = *stop;
-            const int j0 = rowStart[rs];
-            const int j1 = rowStart[rs + 1];
-            // the old y only where it is added to (element 0 otherwise)
-            T yi[NCH];
-#pragma unroll
-            for (int c = 0; c < NCH; c++)
+            if constexpr (kChannelLanes<NCH>)
             {
-                yi[c] = y[accumulate ? static_cast<long>(rs) * NCH + c : 0];
-            }
-            if (stopped)
-            {
+                const int t = blockIdx.x * kBlock + threadIdx.x;
+                const int row = t / L;
+                const bool valid = row < rows;
+                const int rs = valid ? row : 0;
+                const int stopped = *stop;
+                const int j0 = rowStart[rs];
+                const int j1 = rowStart[rs + 1];
+                const long i = static_cast<long>(rs) * NCH + t % NCH;
+                const T yi = y[accumulate ? i : 0];
+                const T inv = xInit ? initInv[rs] : T(0);
+                if (stopped)
+                {
+                    return;
+                }
+                const McgsMatrix<T> M{rows, rowStart, nullptr, column, values, nullptr, nullptr};
+                const T s = rowDotChannels<T, L, NCH>(M, j0, valid ? j1 : j0, x);
+                if (valid && t % L < NCH)
+                {
+                    y[i] = accumulate ? yi + s : s;
+                    if (xInit)
+                    {
+                        xInit[i] = (initScale * inv) * s;
+                    }
+                }
                 return;
             }
-            const McgsMatrix<T> M{rows, rowStart, nullptr, column, values, nullptr, nullptr};
-            T s[NCH];
-            rowDot<T, L, NCH>(M, j0, valid ? j1 : j0, x, s);
-            if (valid && lane == 0)
+            else
             {
+                const int t = blockIdx.x * kBlock + threadIdx.x;
+                const int row = t / L;
+                const int lane = t % L;
+                const bool valid = row < rows;
+                const int rs = valid ? row : 0;
+                const int stopped = *stop;
+                const int j0 = rowStart[rs];
+                const int j1 = rowStart[rs + 1];
+                // the old y only where it is added to (element 0 otherwise)
+                T yi[NCH];
 #pragma unroll
                 for (int c = 0; c < NCH; c++)
                 {
-                    y[static_cast<long>(row) * NCH + c] = accumulate ? yi[c] + s[c] : s[c];
+                    yi[c] = y[accumulate ? static_cast<long>(rs) * NCH + c : 0];
                 }
-                if (xInit)
+                if (stopped)
                 {
-                    const T scale = initScale * initInv[row];
+                    return;
+                }
+                const McgsMatrix<T> M{rows, rowStart, nullptr, column, values, nullptr, nullptr};
+                T s[NCH];
+                rowDot<T, L, NCH>(M, j0, valid ? j1 : j0, x, s);
+                if (valid && lane == 0)
+                {
 #pragma unroll
                     for (int c = 0; c < NCH; c++)
                     {
-                        xInit[static_cast<long>(row) * NCH + c] = scale * s[c];
+                        y[static_cast<long>(row) * NCH + c] = accumulate ? yi[c] + s[c] : s[c];
+                    }
+                    if (xInit)
+                    {
+                        const T scale = initScale * initInv[row];
+#pragma unroll
+                        for (int c = 0; c < NCH; c++)
+                        {
+                            xInit[static_cast<long>(row) * NCH + c] = scale * s[c];
+                        }
                     }
                 }
             }
@@ -177,43 +304,76 @@ namespace nsfem
         __global__ void __launch_bounds__(kBlock) amgChebKernel(McgsMatrix<T> A, const T * __restrict__ b, const T * xIn, const T * dIn,
                                                                 T * __restrict__ xOut, T * dOut, T c1, T c2, const int * __restrict__ stop)
         {
-            const int t = blockIdx.x * kBlock + threadIdx.x;
-            const int row = t / L;
-            const int lane = t % L;
-            const bool valid = row < A.n;
-            const int rs = valid ? row : 0;
-            const int stopped = *stop;
-            const int j0 = A.rowStart[rs];
-            const int j1 = A.rowStart[rs + 1];
-            const T dg = A.diag[rs];
-            const T inv = A.invDiag[rs];
-            T bi[NCH], xi[NCH], di[NCH];
-#pragma unroll
-            for (int c = 0; c < NCH; c++)
+            if constexpr (kChannelLanes<NCH>)
             {
-                const long i = static_cast<long>(rs) * NCH + c;
-                bi[c] = b[i];
-                xi[c] = xIn[i];
-                di[c] = dIn[i];
-            }
-            if (stopped | (j1 < j0))
-            {
-                return; // j1 < j0 never holds (see amgSweepKernel)
-            }
-            T s[NCH];
-            rowDot<T, L, NCH>(A, j0, valid ? j1 : j0, xIn, s);
-            if (valid && lane == 0)
-            {
-#pragma unroll
-                for (int c = 0; c < NCH; c++)
+                const int t = blockIdx.x * kBlock + threadIdx.x;
+                const int row = t / L;
+                const bool valid = row < A.n;
+                const int rs = valid ? row : 0;
+                const int stopped = *stop;
+                const int j0 = A.rowStart[rs];
+                const int j1 = A.rowStart[rs + 1];
+                const T dg = A.diag[rs];
+                const T inv = A.invDiag[rs];
+                const long i = static_cast<long>(rs) * NCH + t % NCH;
+                const T bi = b[i], xi = xIn[i], di = dIn[i];
+                if (stopped | (j1 < j0))
                 {
-                    const long i = static_cast<long>(row) * NCH + c;
-                    const T r = bi[c] - fmaT(dg, xi[c], s[c]);
-                    const T d = fmaT(c1, di[c], c2 * (inv * r));
-                    xOut[i] = xi[c] + d;
+                    return;
+                }
+                const T s = rowDotChannels<T, L, NCH>(A, j0, valid ? j1 : j0, xIn);
+                if (valid && t % L < NCH)
+                {
+                    const T r = bi - fmaT(dg, xi, s);
+                    const T d = fmaT(c1, di, c2 * (inv * r));
+                    xOut[i] = xi + d;
                     if (dOut)
                     {
                         dOut[i] = d;
+                    }
+                }
+                return;
+            }
+            else
+            {
+                const int t = blockIdx.x * kBlock + threadIdx.x;
+                const int row = t / L;
+                const int lane = t % L;
+                const bool valid = row < A.n;
+                const int rs = valid ? row : 0;
+                const int stopped = *stop;
+                const int j0 = A.rowStart[rs];
+                const int j1 = A.rowStart[rs + 1];
+                const T dg = A.diag[rs];
+                const T inv = A.invDiag[rs];
+                T bi[NCH], xi[NCH], di[NCH];
+#pragma unroll
+                for (int c = 0; c < NCH; c++)
+                {
+                    const long i = static_cast<long>(rs) * NCH + c;
+                    bi[c] = b[i];
+                    xi[c] = xIn[i];
+                    di[c] = dIn[i];
+                }
+                if (stopped | (j1 < j0))
+                {
+                    return; // j1 < j0 never holds (see amgSweepKernel)
+                }
+                T s[NCH];
+                rowDot<T, L, NCH>(A, j0, valid ? j1 : j0, xIn, s);
+                if (valid && lane == 0)
+                {
+#pragma unroll
+                    for (int c = 0; c < NCH; c++)
+                    {
+                        const long i = static_cast<long>(row) * NCH + c;
+                        const T r = bi[c] - fmaT(dg, xi[c], s[c]);
+                        const T d = fmaT(c1, di[c], c2 * (inv * r));
+                        xOut[i] = xi[c] + d;
+                        if (dOut)
+                        {
+                            dOut[i] = d;
+                        }
                     }
                 }
             }
@@ -237,33 +397,43 @@ namespace nsfem
             }
         }
 
-        // x = Ainv b on the coarsest level (dense, row-major): one wavefront per row.
+        // x = Ainv b on the coarsest level: the inverse dense, row-major, ld x
+        // ld with zeros past n (ld a multiple of 64), b zero past n.  Bound by
+        // reading the inverse.  Up to four channels: one wavefront per row,
+        // four entries a lane and step.
         template <typename T, int NCH>
-        __global__ void __launch_bounds__(kBlock) amgDenseKernel(int n, const T * __restrict__ inv, const T * __restrict__ b,
+        __global__ void __launch_bounds__(kBlock) amgDenseKernel(int n, int ld, const T * __restrict__ inv, const T * __restrict__ b,
                                                                  T * __restrict__ x, const int * __restrict__ stop)
         {
-            if (*stop)
+            const int row = (blockIdx.x * kBlock + threadIdx.x) >> 6;
+            if (*stop || row >= n)
             {
                 return;
             }
-            const int row = (blockIdx.x * kBlock + threadIdx.x) >> 6;
             const int lane = threadIdx.x & 63;
+            const T * a = inv + static_cast<size_t>(row) * ld;
             T s[NCH];
 #pragma unroll
             for (int c = 0; c < NCH; c++)
             {
                 s[c] = 0;
             }
-            if (row < n)
+#pragma unroll 4
+            for (int j = 4 * lane; j < ld; j += 256)
             {
-                const T * a = inv + static_cast<size_t>(row) * n;
-                for (int j = lane; j < n; j += 64)
+                T v[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++)
                 {
-                    const T v = a[j];
+                    v[u] = a[j + u];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                {
 #pragma unroll
                     for (int c = 0; c < NCH; c++)
                     {
-                        s[c] = fmaT(v, b[static_cast<long>(j) * NCH + c], s[c]);
+                        s[c] = fmaT(v[u], b[static_cast<long>(j + u) * NCH + c], s[c]);
                     }
                 }
             }
@@ -272,13 +442,74 @@ namespace nsfem
             {
                 s[c] = laneGroupSum<64>(s[c]);
             }
-            if (row < n && lane == 0)
+            if (lane == 0)
             {
 #pragma unroll
                 for (int c = 0; c < NCH; c++)
                 {
                     x[static_cast<long>(row) * NCH + c] = s[c];
                 }
+            }
+        }
+
+        // 8 and 16 channels: sixteen rows a workgroup on the matrix cores (a
+        // vector form reads b once per row: 1,008 rows x 16 channels would
+        // move 65 MB of it for 4 MB of inverse).  A wave takes every fourth
+        // stretch of 16 columns; lane l holds row l % 16 and, as the tile's
+        // column, channel l % 16, both at inner indices 4 (l / 16) + u.  The
+        // four waves' tiles are added in wave order.
+        template <typename T, int NCH>
+        __global__ void __launch_bounds__(kBlock) amgDenseTileKernel(int n, int ld, const T * __restrict__ inv, const T * __restrict__ b,
+                                                                     T * __restrict__ x, const int * __restrict__ stop)
+        {
+            typedef T Tile __attribute__((ext_vector_type(4)));
+            __shared__ T sm[4][16][17];
+            if (*stop)
+            {
+                return;
+            }
+            const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+            const int i = lane & 15, g = lane >> 4;
+            const int r0 = blockIdx.x * 16;
+            const T * a = inv + static_cast<size_t>(r0 + i) * ld + 4 * g;
+            const int c = i < NCH ? i : 0;
+            Tile acc = {T(0), T(0), T(0), T(0)};
+#pragma unroll 2
+            for (int k0 = 16 * wave; k0 < ld; k0 += 64)
+            {
+                T av[4], bv[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                {
+                    av[u] = a[k0 + u];
+                    bv[u] = b[static_cast<long>(k0 + 4 * g + u) * NCH + c];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                {
+                    const T bu = i < NCH ? bv[u] : T(0);
+                    if constexpr (std::is_same_v<T, float>)
+                    {
+                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u], bu, acc, 0, 0, 0);
+                    }
+                    else
+                    {
+                        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u], bu, acc, 0, 0, 0);
+                    }
+                }
+            }
+            // result rows: 4 (l / 16) + u in FP32, l / 16 + 4 u in FP64
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+            {
+                const int r = std::is_same_v<T, float> ? 4 * g + u : g + 4 * u;
+                sm[wave][r][i] = acc[u];
+            }
+            __syncthreads();
+            const int t = threadIdx.x, r = t >> 4, cc = t & 15;
+            if (r0 + r < n && cc < NCH)
+            {
+                x[static_cast<long>(r0 + r) * NCH + cc] = ((sm[0][r][cc] + sm[1][r][cc]) + sm[2][r][cc]) + sm[3][r][cc];
             }
         }
 
@@ -318,14 +549,68 @@ namespace nsfem
             }
         }
 
+        // Per-channel block sums of a value per thread, channel threadIdx.x % NCH
+        // -> this block's partials.
+        template <int NCH, int W = kWaves>
+        __device__ __forceinline__ void storeChannelParts(double v, double * parts, double * sm)
+        {
+            const double total = channelBlockSum<NCH, W>(v, sm);
+            storeChannelPartial<NCH, NCH>(total, parts, blockIdx.x, 0);
+        }
+
         // r = b - A x (x = 0 and r = b for a zero guess), the V-cycle's copy
-        // of r, per-channel partials of |b|^2 and |r|^2.
+        // of r, the first colour's start of the forward sweep z = r / d
+        // (rows below c0End), per-channel partials of |b|^2 and |r|^2.
         template <typename P, int L, int NCH>
         __global__ void __launch_bounds__(kBlock) amgInitKernel(McgsMatrix<double> A, const double * __restrict__ b, double * __restrict__ x,
-                                                                double * __restrict__ r, P * __restrict__ rP, int zeroGuess, AmgState st)
+                                                                double * __restrict__ r, P * __restrict__ rP, int zeroGuess, AmgState st,
+                                                                P * __restrict__ z, const P * __restrict__ invDiag, int c0End)
         {
             __shared__ double sm[2 * NCH * kWaves];
             constexpr int G = kBlock / L;
+            if constexpr (kChannelLanes<NCH>)
+            {
+                const int c = threadIdx.x % NCH;
+                double bb = 0, rr = 0;
+                for (int base = blockIdx.x * G; base < A.n; base += gridDim.x * G)
+                {
+                    const int row = base + static_cast<int>(threadIdx.x) / L;
+                    const bool valid = row < A.n;
+                    const int rs = valid ? row : base;
+                    const long i = static_cast<long>(rs) * NCH + c;
+                    const double bi = b[i];
+                    double ri = bi;
+                    if (!zeroGuess)
+                    {
+                        const int j0 = A.rowStart[rs];
+                        const int j1 = A.rowStart[rs + 1];
+                        const double s = rowDotChannels<double, L, NCH>(A, j0, valid ? j1 : j0, x);
+                        ri = bi - fmaT(A.diag[rs], x[i], s);
+                    }
+                    if (valid && threadIdx.x % L < NCH)
+                    {
+                        if (zeroGuess)
+                        {
+                            x[i] = 0;
+                        }
+                        r[i] = ri;
+                        const P rp = static_cast<P>(ri);
+                        if constexpr (!std::is_same_v<P, double>)
+                        {
+                            rP[i] = rp;
+                        }
+                        if (row < c0End)
+                        {
+                            z[i] = rp * invDiag[row];
+                        }
+                        bb = fmaT(bi, bi, bb);
+                        rr = fmaT(ri, ri, rr);
+                    }
+                }
+                storeChannelParts<NCH>(bb, st.partBb, sm);
+                storeChannelParts<NCH>(rr, st.partRr, sm);
+                return;
+            }
             const int lane = threadIdx.x % L;
             double bb[NCH], rr[NCH];
 #pragma unroll
@@ -378,9 +663,14 @@ namespace nsfem
                             ri = bi - fmaT(d, x[i], s[c]);
                         }
                         r[i] = ri;
+                        const P rp = static_cast<P>(ri);
                         if constexpr (!std::is_same_v<P, double>)
                         {
-                            rP[i] = static_cast<P>(ri);
+                            rP[i] = rp;
+                        }
+                        if (row < c0End)
+                        {
+                            z[i] = rp * invDiag[row];
                         }
                         bb[c] = fmaT(bi, bi, bb[c]);
                         rr[c] = fmaT(ri, ri, rr[c]);
@@ -427,16 +717,51 @@ namespace nsfem
 
         // beta = rho / rho_before (0 on the first direction and for stopped
         // channels); p = z + beta p, q = A z + beta q (= A p, as
-        // A p_before = q), per-channel partials of p.q.
+        // A p_before = q), per-channel partials of p.q.  A zero beta takes p = z
+        // and q = A z whatever p and q hold (fresh memory, or what a solve
+        // that broke down left).
         template <typename P, int L, int NCH>
-        __global__ void __launch_bounds__(kBlock) amgDirectionKernel(McgsMatrix<double> A, const P * __restrict__ z, double * __restrict__ p,
+        __global__ void __launch_bounds__(kCgBlock<NCH>) amgDirectionKernel(McgsMatrix<double> A, const P * __restrict__ z, double * __restrict__ p,
                                                                      double * __restrict__ q, AmgState st)
         {
             if (st.ints[0])
             {
                 return;
             }
-            __shared__ double sm[NCH * kWaves];
+            __shared__ double sm[NCH * (kCgBlock<NCH> / 64)];
+            if constexpr (kChannelLanes<NCH>)
+            {
+                constexpr int G = kCgBlock<NCH> / L;
+                const int c = threadIdx.x % NCH;
+                const double before = st.scal[NCH + c];
+                const double beta = (st.active[c] && before != 0) ? st.scal[c] / before : 0.0;
+                double acc = 0;
+                for (int base = blockIdx.x * G; base < A.n; base += gridDim.x * G)
+                {
+                    const int row = base + static_cast<int>(threadIdx.x) / L;
+                    const bool valid = row < A.n;
+                    const int rs = valid ? row : base;
+                    const int j0 = A.rowStart[rs];
+                    const int j1 = A.rowStart[rs + 1];
+                    const long i = static_cast<long>(rs) * NCH + c;
+                    const double d = A.diag[rs];
+                    const P zr = z[i];
+                    const double pr = p[i], qr = q[i];
+                    const double s = rowDotChannels<double, L, NCH>(A, j0, valid ? j1 : j0, z);
+                    if (valid && threadIdx.x % L < NCH)
+                    {
+                        const double zi = static_cast<double>(zr);
+                        const double az = fmaT(d, zi, s);
+                        const double pi = beta == 0 ? zi : fmaT(beta, pr, zi);
+                        const double qi = beta == 0 ? az : fmaT(beta, qr, az);
+                        p[i] = pi;
+                        q[i] = qi;
+                        acc = fmaT(pi, qi, acc);
+                    }
+                }
+                storeChannelParts<NCH, kCgBlock<NCH> / 64>(acc, st.partPq, sm);
+                return;
+            }
             double beta[NCH];
 #pragma unroll
             for (int c = 0; c < NCH; c++)
@@ -473,8 +798,9 @@ namespace nsfem
                     {
                         const long i = static_cast<long>(row) * NCH + c;
                         const double zi = static_cast<double>(z[i]);
-                        const double pi = fmaT(beta[c], p[i], zi);
-                        const double qi = fmaT(beta[c], q[i], fmaT(d, zi, s[c]));
+                        const double az = fmaT(d, zi, s[c]);
+                        const double pi = beta[c] == 0 ? zi : fmaT(beta[c], p[i], zi);
+                        const double qi = beta[c] == 0 ? az : fmaT(beta[c], q[i], az);
                         p[i] = pi;
                         q[i] = qi;
                         acc[c] = fmaT(pi, qi, acc[c]);
@@ -487,55 +813,53 @@ namespace nsfem
 
         // alpha = rho / p.q for the channels still iterating, 0 for the
         // stopped ones (every block sums the partials itself, in the same
-        // order); x += alpha p, r -= alpha q, the V-cycle's copy of r,
-        // per-channel partials of |r|^2.
+        // order); x += alpha p, r -= alpha q, the V-cycle's copy of r, the
+        // first colour's start of the forward sweep z = r / d (rows below
+        // c0End), per-channel partials of |r|^2.  Flat over the interleaved
+        // elements: a thread keeps one channel.
         template <typename P, int NCH>
-        __global__ void __launch_bounds__(kBlock) amgUpdateKernel(int n, const double * __restrict__ p, const double * __restrict__ q,
+        __global__ void __launch_bounds__(kCgBlock<NCH>) amgUpdateKernel(int n, const double * __restrict__ p, const double * __restrict__ q,
                                                                   double * __restrict__ x, double * __restrict__ r, P * __restrict__ rP,
-                                                                  AmgState st)
+                                                                  AmgState st, P * __restrict__ z, const P * __restrict__ invDiag, int c0End)
         {
             if (st.ints[0])
             {
                 return;
             }
-            __shared__ double sm[NCH * kWaves];
+            constexpr int BLOCK = kCgBlock<NCH>;
+            __shared__ double sm[NCH * (BLOCK / 64)];
             __shared__ double shAlpha[NCH];
-            double pq[NCH];
-            sumParts<NCH>(st.partPq, st.parts, pq, sm);
-            if (threadIdx.x == 0)
+            const int t = threadIdx.x;
+            const int act = t < NCH ? st.active[t] : 0;
+            const double rho = t < NCH ? st.scal[t] : 0.0;
+            const double pq = channelPartialSum<NCH, BLOCK>(st.partPq, st.parts, sm);
+            if (t < NCH)
             {
-#pragma unroll
-                for (int c = 0; c < NCH; c++)
-                {
-                    shAlpha[c] = st.active[c] ? st.scal[c] / pq[c] : 0.0;
-                }
+                shAlpha[t] = act ? rho / pq : 0.0;
             }
             __syncthreads();
-            double alpha[NCH], acc[NCH];
-#pragma unroll
-            for (int c = 0; c < NCH; c++)
+            const double alpha = shAlpha[t % NCH];
+            double acc = 0;
+            const long end = static_cast<long>(n) * NCH, stride = static_cast<long>(gridDim.x) * BLOCK;
+#pragma unroll 2
+            for (long i = static_cast<long>(blockIdx.x) * BLOCK + t; i < end; i += stride)
             {
-                alpha[c] = shAlpha[c];
-                acc[c] = 0;
-            }
-            for (int row = blockIdx.x * kBlock + threadIdx.x; row < n; row += gridDim.x * kBlock)
-            {
-#pragma unroll
-                for (int c = 0; c < NCH; c++)
+                x[i] = fmaT(alpha, p[i], x[i]);
+                const double ri = fmaT(-alpha, q[i], r[i]);
+                r[i] = ri;
+                const P rp = static_cast<P>(ri);
+                if constexpr (!std::is_same_v<P, double>)
                 {
-                    const long i = static_cast<long>(row) * NCH + c;
-                    x[i] = fmaT(alpha[c], p[i], x[i]);
-                    const double ri = fmaT(-alpha[c], q[i], r[i]);
-                    r[i] = ri;
-                    if constexpr (!std::is_same_v<P, double>)
-                    {
-                        rP[i] = static_cast<P>(ri);
-                    }
-                    acc[c] = fmaT(ri, ri, acc[c]);
+                    rP[i] = rp;
                 }
+                const int row = static_cast<int>(i / NCH);
+                if (row < c0End)
+                {
+                    z[i] = rp * invDiag[row];
+                }
+                acc = fmaT(ri, ri, acc);
             }
-            blockSum<NCH>(acc, sm);
-            storeParts<NCH>(acc, st.partRr);
+            storeChannelParts<NCH, BLOCK / 64>(acc, st.partRr, sm);
         }
 
         // per-channel partials of r.z
@@ -547,88 +871,173 @@ namespace nsfem
                 return;
             }
             __shared__ double sm[NCH * kWaves];
-            double acc[NCH];
+            double acc = 0;
+            const long end = static_cast<long>(n) * NCH, stride = static_cast<long>(gridDim.x) * kBlock;
+            for (long i = static_cast<long>(blockIdx.x) * kBlock + threadIdx.x; i < end; i += stride)
+            {
+                acc = fmaT(r[i], static_cast<double>(z[i]), acc);
+            }
+            storeChannelParts<NCH>(acc, st.partRho, sm);
+        }
+
+        // The backward sweep's last colour (rows below c0End, full rows) fused
+        // with the partials of r.z over all rows, whose other colours are final
+        // (one launch fewer; every block takes a share of both).
+        template <typename P, int L, int NCH>
+        __global__ void __launch_bounds__(kCgBlock<NCH>) amgSweepRhoKernel(McgsMatrix<P> A, int c0End, const P * __restrict__ b, P * __restrict__ x,
+                                                                    const double * __restrict__ r, AmgState st)
+        {
+            if (st.ints[0])
+            {
+                return;
+            }
+            constexpr int BLOCK = kCgBlock<NCH>, G = BLOCK / L;
+            __shared__ double sm[NCH * (BLOCK / 64)];
+            double acc = 0; // of channel threadIdx.x % NCH
+            double lead[NCH]; // lane-split rows: all channels on the row's first lane
 #pragma unroll
             for (int c = 0; c < NCH; c++)
             {
-                acc[c] = 0;
+                lead[c] = 0;
             }
-            for (int row = blockIdx.x * kBlock + threadIdx.x; row < n; row += gridDim.x * kBlock)
+            for (int base = blockIdx.x * G; base < c0End; base += gridDim.x * G)
+            {
+                const int row = base + static_cast<int>(threadIdx.x) / L;
+                const bool valid = row < c0End;
+                const int rs = valid ? row : base;
+                const int j0 = A.rowStart[rs];
+                const int j1 = A.rowStart[rs + 1];
+                const P d = A.invDiag[rs];
+                if constexpr (kChannelLanes<NCH>)
+                {
+                    const long i = static_cast<long>(rs) * NCH + threadIdx.x % NCH;
+                    const P bi = b[i];
+                    const double ri = r[i];
+                    const P s = rowDotChannels<P, L, NCH>(A, j0, valid ? j1 : j0, x);
+                    if (valid && threadIdx.x % L < NCH)
+                    {
+                        const P xi = (bi - s) * d;
+                        x[i] = xi;
+                        acc = fmaT(ri, static_cast<double>(xi), acc);
+                    }
+                }
+                else
+                {
+                    P bi[NCH], s[NCH];
+                    double ri[NCH];
+#pragma unroll
+                    for (int c = 0; c < NCH; c++)
+                    {
+                        const long i = static_cast<long>(rs) * NCH + c;
+                        bi[c] = b[i];
+                        ri[c] = r[i];
+                    }
+                    rowDot<P, L, NCH>(A, j0, valid ? j1 : j0, x, s);
+                    if (valid && threadIdx.x % L == 0)
+                    {
+#pragma unroll
+                        for (int c = 0; c < NCH; c++)
+                        {
+                            const P xi = (bi[c] - s[c]) * d;
+                            x[static_cast<long>(row) * NCH + c] = xi;
+                            lead[c] = fmaT(ri[c], static_cast<double>(xi), lead[c]);
+                        }
+                    }
+                }
+            }
+            const long end = static_cast<long>(A.n) * NCH, stride = static_cast<long>(gridDim.x) * BLOCK;
+#pragma unroll 2
+            for (long i = static_cast<long>(c0End) * NCH + static_cast<long>(blockIdx.x) * BLOCK + threadIdx.x; i < end; i += stride)
+            {
+                acc = fmaT(r[i], static_cast<double>(x[i]), acc);
+            }
+            if constexpr (kChannelLanes<NCH>)
+            {
+                storeChannelParts<NCH, BLOCK / 64>(acc, st.partRho, sm);
+            }
+            else
             {
 #pragma unroll
                 for (int c = 0; c < NCH; c++)
                 {
-                    const long i = static_cast<long>(row) * NCH + c;
-                    acc[c] = fmaT(r[i], static_cast<double>(z[i]), acc[c]);
+                    lead[c] += static_cast<int>(threadIdx.x) % NCH == c ? acc : 0.0;
                 }
+                blockSum<NCH>(lead, sm);
+                storeParts<NCH>(lead, st.partRho);
             }
-            blockSum<NCH>(acc, sm);
-            storeParts<NCH>(acc, st.partRho);
         }
 
         // rho = r.z per channel; after an update (init = 0) also |r|^2, the
         // iteration count and each channel's stopping test.  A channel still
         // iterating with r.z <= 0 (a breakdown) or a non-finite value stops
         // the solve as non-finite; the solve stops when no channel iterates.
+        // Thread c handles channel c; its state loads with the partials.
         template <int NCH>
-        __global__ void __launch_bounds__(kBlock) amgFinalizeKernel(AmgState st, int init)
+        __global__ void __launch_bounds__(kFinBlock) amgFinalizeKernel(AmgState st, int init)
         {
-            if (st.ints[0])
+            __shared__ double sm[2 * NCH * kFinWaves];
+            constexpr int G = kFinBlock / NCH;
+            const int t = threadIdx.x, c = t % NCH;
+            const int stopped = st.ints[0];
+            const int iters = st.ints[1];
+            const int was = t < NCH ? st.active[t] : 0;
+            const double rhoOld = t < NCH ? st.scal[t] : 0.0;
+            const double bb = t < NCH ? st.scal[2 * NCH + t] : 0.0;
+            double rho = 0, rr = 0;
+#pragma unroll 4
+            for (int k = t / NCH; k < st.parts; k += G)
+            {
+                rho += st.partRho[static_cast<size_t>(k) * NCH + c];
+                rr += st.partRr[static_cast<size_t>(k) * NCH + c];
+            }
+            if (stopped)
             {
                 return;
             }
-            __shared__ double sm[NCH * kWaves];
-            double rho[NCH], rr[NCH];
-            sumParts<NCH>(st.partRho, st.parts, rho, sm);
-            if (!init)
+            channelBlockSum2<NCH, kFinWaves>(rho, rr, sm);
+            if (st.tol2 < 0)
             {
-                sumParts<NCH>(st.partRr, st.parts, rr, sm);
+                // kernel timing: never stops, whatever the vectors hold
+                if (t < NCH)
+                {
+                    st.scal[NCH + t] = rhoOld;
+                    st.scal[t] = std::isfinite(rho) && rho > 0 ? rho : 1.0;
+                }
+                return;
             }
-            if (threadIdx.x == 0)
+            int act = was, bad = 0;
+            if (t < NCH)
             {
-                if (st.tol2 < 0)
-                {
-                    // kernel timing: never stops, whatever the vectors hold
-#pragma unroll
-                    for (int c = 0; c < NCH; c++)
-                    {
-                        st.scal[NCH + c] = st.scal[c];
-                        st.scal[c] = std::isfinite(rho[c]) && rho[c] > 0 ? rho[c] : 1.0;
-                    }
-                    return;
-                }
-                int any = 0, bad = 0;
-#pragma unroll
-                for (int c = 0; c < NCH; c++)
-                {
-                    int act = st.active[c];
-                    if (!init)
-                    {
-                        st.scal[3 * NCH + c] = rr[c];
-                        if (act)
-                        {
-                            if (!std::isfinite(rr[c]))
-                            {
-                                bad = 1;
-                            }
-                            else if (rr[c] <= st.tol2 * st.scal[2 * NCH + c])
-                            {
-                                act = 0;
-                            }
-                        }
-                    }
-                    if (act && (!std::isfinite(rho[c]) || !(rho[c] > 0)))
-                    {
-                        bad = 1;
-                    }
-                    st.active[c] = act;
-                    any |= act;
-                    st.scal[NCH + c] = init ? 0.0 : st.scal[c];
-                    st.scal[c] = rho[c];
-                }
                 if (!init)
                 {
-                    st.ints[1] += 1;
+                    st.scal[3 * NCH + t] = rr;
+                    if (act)
+                    {
+                        if (!std::isfinite(rr))
+                        {
+                            bad = 1;
+                        }
+                        else if (rr <= st.tol2 * bb)
+                        {
+                            act = 0;
+                        }
+                    }
+                }
+                if (act && (!std::isfinite(rho) || !(rho > 0)))
+                {
+                    bad = 1;
+                }
+                st.active[t] = act;
+                st.scal[NCH + t] = init ? 0.0 : rhoOld;
+                st.scal[t] = rho;
+            }
+            const int any = __syncthreads_or(act);
+            bad = __syncthreads_or(bad);
+            if (t == 0)
+            {
+                if (!init)
+                {
+                    st.ints[1] = iters + 1;
                 }
                 st.ints[0] = bad ? 2 : (any ? 0 : 1);
             }
@@ -660,12 +1069,60 @@ namespace nsfem
             }
         }
 
+        // f<L>(): lanes per row; four channels or more take NCH lanes per
+        // group and as many groups as keep a mean row to one or two rounds
+        template <int NCH, typename F>
+        void byRowLanes(int lanes, double meanRow, F && f)
+        {
+            if constexpr (kChannelLanes<NCH>)
+            {
+                if (meanRow < 4)
+                {
+                    f.template operator()<NCH>();
+                }
+                else if (meanRow < 10 || 4 * NCH > 64)
+                {
+                    f.template operator()<2 * NCH>();
+                }
+                else
+                {
+                    f.template operator()<4 * NCH>();
+                }
+            }
+            else
+            {
+                byLanes(lanes, f);
+            }
+        }
+
         int lanesFor(double meanRow) { return std::max(2, std::min(16, lanesForMeanRow(meanRow))); }
+        // A level's own rows: two lanes take eight entries in one round of
+        // loads, and every lane works (P1 rows of six entries, 500k rows, FP32
+        // V-cycle: 130 us an iteration, 135 on four lanes, 159 on eight; the
+        // direction kernel 15.1, 17.1 and 27.8 us).  Longer rows (the coarse
+        // levels' 17 entries) measure the same on 4 to 16 lanes.
+        int levelLanes(double meanRow) { return meanRow <= 8 ? 2 : lanesFor(meanRow); }
         double meanRow(const std::vector<int> & rowStart)
         {
             const int rows = static_cast<int>(rowStart.size()) - 1;
             return rows > 0 ? static_cast<double>(rowStart.back()) / rows : 1.0;
         }
+    } // namespace
+
+    namespace
+    {
+        // The coarsest level is the first one (never a finest level of more
+        // than 512 rows) whose dense inverse is small enough, computed on the
+        // GPU: one launch that reads it takes less than the eight launches and
+        // the deeper levels that it replaces, some 3.3 us each.  Up to 100 MB
+        // (5,120 rows in FP32, 3,620 in FP64) it stays in the Infinity Cache.
+        // Measured per CG iteration against 512 rows: 60k rows FP64 78.9 ->
+        // 66.4 us, 300k FP64 (2,700 coarse rows) 120 -> 111, 500k FP32 (4,624)
+        // 129.6 -> 124.8, 100k x 16 FP32 (1,008) 170 -> 157.  Four channels or
+        // more do that many times the arithmetic per entry: 40k x 8 FP32 with
+        // 4,400 coarse rows took 105 us against 89 with 432.
+        constexpr long kCoarseBytes = 100L << 20;
+        constexpr int kMaxCoarseWide = 2432;
     } // namespace
 
     AmgPcg::AmgPcg(const CsrD & stripped, const std::vector<int> & rowSplit, const std::vector<double> & diag,
@@ -678,7 +1135,40 @@ namespace nsfem
             throw std::invalid_argument("amg_pcg solves 1, 2, 4, 8 or 16 right-hand sides");
         }
         const auto t0 = std::chrono::steady_clock::now();
-        const AmgHierarchy h = buildAmgHierarchy(stripped, rowSplit, diag, colorStart);
+        const int maxCoarse = nch_ >= 4 ? kMaxCoarseWide
+                                        : static_cast<int>(std::sqrt(static_cast<double>(kCoarseBytes) / (mixed_ ? 4 : 8)));
+        AmgHierarchy h;
+        bool inverted = false;
+        if (n_ > AmgOptions{}.maxCoarse)
+        {
+            AmgOptions opt;
+            opt.maxCoarse = std::min(maxCoarse, n_ - 1);
+            opt.invertCoarse = false;
+            h = buildAmgHierarchy(stripped, rowSplit, diag, colorStart, opt);
+            if (h.levels.back().n <= maxCoarse)
+            {
+                coarseN_ = h.levels.back().n;
+                coarseLd_ = (coarseN_ + 63) / 64 * 64;
+                const size_t entries = static_cast<size_t>(coarseLd_) * coarseLd_;
+                if (mixed_)
+                {
+                    coarse32_.resize(entries);
+                    inverted = denseInverseGpu<float>(coarseN_, h.coarseMatrix, coarseLd_, coarse32_.get(), s);
+                }
+                else
+                {
+                    coarse64_.resize(entries);
+                    inverted = denseInverseGpu<double>(coarseN_, h.coarseMatrix, coarseLd_, coarse64_.get(), s);
+                }
+            }
+        }
+        if (!inverted)
+        {
+            // small systems, coarsening that stalls, and operators that are not
+            // definite on that level: down to 512 rows, inverted (or
+            // rejected) on the host
+            h = buildAmgHierarchy(stripped, rowSplit, diag, colorStart);
+        }
         complexity_ = h.operatorComplexity;
         levels_.resize(h.levels.size());
         const size_t ts = mixed_ ? 4 : 8;
@@ -690,7 +1180,7 @@ namespace nsfem
             L.n = H.n;
             L.colorStart = H.colorStart;
             L.lambdaMax = H.lambdaMax;
-            L.lanes = lanesFor(meanRow(H.stripped.rowStart));
+            L.lanes = levelLanes(meanRow(H.stripped.rowStart));
             L.nnz = H.stripped.nnz();
             for (int i = 0; i < H.n; i++)
             {
@@ -747,23 +1237,43 @@ namespace nsfem
                 }
             }
         }
-        coarseN_ = h.levels.back().n;
-        if (mixed_)
+        if (!inverted)
         {
-            coarse32_.upload(std::vector<float>(h.coarseInverse.begin(), h.coarseInverse.end()));
+            coarseN_ = h.levels.back().n;
+            coarseLd_ = (coarseN_ + 63) / 64 * 64;
+            std::vector<double> padded(static_cast<size_t>(coarseLd_) * coarseLd_, 0.0);
+            for (int i = 0; i < coarseN_; i++)
+            {
+                std::copy(h.coarseInverse.begin() + static_cast<size_t>(i) * coarseN_,
+                          h.coarseInverse.begin() + static_cast<size_t>(i + 1) * coarseN_, padded.begin() + static_cast<size_t>(i) * coarseLd_);
+            }
+            if (mixed_)
+            {
+                coarse32_.upload(std::vector<float>(padded.begin(), padded.end()));
+            }
+            else
+            {
+                coarse64_.upload(padded);
+            }
         }
-        else
         {
-            coarse64_.upload(h.coarseInverse);
+            // the dense product reads whole rows: its right-hand side is
+            // zero past the level's rows
+            Level & C = levels_.back();
+            C.b.resize(static_cast<size_t>(coarseLd_) * vb);
+            C.b.zero();
         }
-        const size_t nv = static_cast<size_t>(n_) * nch_;
-        r_.resize(nv);
+        // (a one-level hierarchy's dense product reads r past its rows, too)
+        const size_t nv = static_cast<size_t>(n_) * nch_, pad = static_cast<size_t>(64) * nch_;
+        r_.resize(nv + pad);
+        r_.zero();
         p_.resize(nv);
         q_.resize(nv);
         z_.resize(nv * ts);
         if (mixed_)
         {
-            rP_.resize(nv * ts);
+            rP_.resize((nv + pad) * ts);
+            rP_.zero();
         }
         parts_ = std::max(1, std::min(1024, (n_ + kBlock - 1) / kBlock));
         scal_.resize(4 * nch_);
@@ -899,6 +1409,11 @@ namespace nsfem
         }
     }
 
+    AmgState AmgPcg::state(double tol2)
+    {
+        return AmgState{scal_.get(), ints_.get(), active_.get(), partPq_.get(), partRr_.get(), partRho_.get(), partBb_.get(), parts_, tol2};
+    }
+
     template <typename T>
     McgsMatrix<T> AmgPcg::levelMatrix(int l) const
     {
@@ -927,7 +1442,7 @@ namespace nsfem
     }
 
     template <typename T, int NCH>
-    void AmgPcg::enqueueVcycle(hipStream_t s, const T * b0, T * x0)
+    void AmgPcg::enqueueVcycle(hipStream_t s, const T * b0, T * x0, bool fused, double tol2)
     {
         const int * stop = ints_.get();
         const int last = numLevels() - 1;
@@ -965,7 +1480,7 @@ namespace nsfem
                 return;
             }
             const McgsMatrix<T> A = levelMatrix<T>(l);
-            byLanes(L.lanes, [&]<int LN>()
+            byRowLanes<NCH>(L.lanes, L.nnz / L.n, [&]<int LN>()
                     { amgSweepKernel<T, LN, NCH><<<grid(r1 - r0, LN), kBlock, 0, s>>>(A, r0, r1, bOf(l), xOf(l), lowerOnly, stop); });
         };
         // Chebyshev levels: the steps alternate between x and xa (other rows
@@ -979,7 +1494,7 @@ namespace nsfem
             const Level & L = levels_[l];
             const McgsMatrix<T> A = levelMatrix<T>(l);
             const T c1 = static_cast<T>(L.chebC1[k]), c2 = static_cast<T>(L.chebC2[k]);
-            byLanes(L.lanes, [&]<int LN>()
+            byRowLanes<NCH>(L.lanes, L.nnz / L.n, [&]<int LN>()
                     { amgChebKernel<T, LN, NCH><<<grid(L.n, LN), kBlock, 0, s>>>(A, bOf(l), xIn, dIn, xOut, dOut, c1, c2, stop); });
         };
         // the current iterate of every level
@@ -990,7 +1505,8 @@ namespace nsfem
             const int deg = L.chebDegree;
             if (deg == 0)
             {
-                for (int c = 0; c < static_cast<int>(L.colorStart.size()) - 1; c++)
+                // (the finest level's first colour starts with the residual's copy)
+                for (int c = fused && l == 0 ? 1 : 0; c < static_cast<int>(L.colorStart.size()) - 1; c++)
                 {
                     sweep(l, c, 1);
                 }
@@ -1018,7 +1534,7 @@ namespace nsfem
             }
             T * r = reinterpret_cast<T *>(L.r.get());
             const McgsMatrix<T> A = levelMatrix<T>(l);
-            byLanes(L.lanes, [&]<int LN>() { amgResidualKernel<T, LN, NCH><<<grid(L.n, LN), kBlock, 0, s>>>(A, bOf(l), cur[l], r, stop); });
+            byRowLanes<NCH>(L.lanes, L.nnz / L.n, [&]<int LN>() { amgResidualKernel<T, LN, NCH><<<grid(L.n, LN), kBlock, 0, s>>>(A, bOf(l), cur[l], r, stop); });
             // the coarser level's first Chebyshev iterate with its right-hand side
             const Level & C = levels_[l + 1];
             const bool init = l + 1 < last && C.chebDegree > 0;
@@ -1029,7 +1545,7 @@ namespace nsfem
             }
             T * cInit = init ? xaOf(l + 1) : nullptr;
             const T cScale = init ? static_cast<T>(C.chebC2[0]) : T(0);
-            byLanes(L.rLanes, [&]<int LN>()
+            byRowLanes<NCH>(L.rLanes, L.nnzR / L.rRows, [&]<int LN>()
                     {
                         amgSpmvKernel<T, LN, NCH><<<grid(L.rRows, LN), kBlock, 0, s>>>(L.rRows, L.rRowStart.get(), L.rColumn.get(), rVals(L),
                                                                                       r, reinterpret_cast<T *>(levels_[l + 1].b.get()), 0,
@@ -1046,13 +1562,20 @@ namespace nsfem
             {
                 inv = coarse32_.get();
             }
-            amgDenseKernel<T, NCH><<<grid(coarseN_, 64), kBlock, 0, s>>>(coarseN_, inv, bOf(last), xOf(last), stop);
+            if constexpr (NCH >= 8)
+            {
+                amgDenseTileKernel<T, NCH><<<(coarseN_ + 15) / 16, kBlock, 0, s>>>(coarseN_, coarseLd_, inv, bOf(last), xOf(last), stop);
+            }
+            else
+            {
+                amgDenseKernel<T, NCH><<<grid(coarseN_, 64), kBlock, 0, s>>>(coarseN_, coarseLd_, inv, bOf(last), xOf(last), stop);
+            }
             cur[last] = xOf(last);
         }
         for (int l = last - 1; l >= 0; l--)
         {
             const Level & L = levels_[l];
-            byLanes(L.pLanes, [&]<int LN>()
+            byRowLanes<NCH>(L.pLanes, L.nnzP / L.pRows, [&]<int LN>()
                     {
                         amgSpmvKernel<T, LN, NCH><<<grid(L.pRows, LN), kBlock, 0, s>>>(L.pRows, L.pRowStart.get(), L.pColumn.get(), pVals(L),
                                                                                       cur[l + 1], cur[l], 1, stop, nullptr, nullptr, T(0));
@@ -1060,9 +1583,16 @@ namespace nsfem
             const int deg = L.chebDegree;
             if (deg == 0)
             {
-                for (int c = static_cast<int>(L.colorStart.size()) - 2; c >= 0; c--)
+                for (int c = static_cast<int>(L.colorStart.size()) - 2; c >= (fused && l == 0 ? 1 : 0); c--)
                 {
                     sweep(l, c, 0);
+                }
+                if (fused && l == 0)
+                {
+                    const McgsMatrix<T> A = levelMatrix<T>(0);
+                    const AmgState st = state(tol2);
+                    byRowLanes<NCH>(L.lanes, L.nnz / L.n, [&]<int LN>()
+                                    { amgSweepRhoKernel<T, LN, NCH><<<parts_, kCgBlock<NCH>, 0, s>>>(A, L.colorStart[1], b0, x0, r_.get(), st); });
                 }
             }
             else
@@ -1086,33 +1616,46 @@ namespace nsfem
     }
 
     template <typename P, int NCH>
+    void AmgPcg::enqueuePrecond(hipStream_t s, const P * rP, P * z, double tol2, int init)
+    {
+        // the V-cycle, r.z and the scalars; a Gauss-Seidel finest level takes
+        // r.z with its last colour
+        enqueueVcycle<P, NCH>(s, rP, z, fusedSweep(), tol2);
+        const AmgState st = state(tol2);
+        if (!fusedSweep())
+        {
+            amgRhoKernel<P, NCH><<<parts_, kBlock, 0, s>>>(n_, r_.get(), z, st);
+        }
+        amgFinalizeKernel<NCH><<<1, kFinBlock, 0, s>>>(st, init);
+        NSFEM_HIP(hipGetLastError());
+    }
+
+    template <typename P, int NCH>
     void AmgPcg::enqueueInit(hipStream_t s, const double * b, double * x, bool zeroGuess, double tol2)
     {
-        const AmgState st{scal_.get(), ints_.get(), active_.get(), partPq_.get(), partRr_.get(), partRho_.get(), partBb_.get(), parts_, tol2};
+        const AmgState st = state(tol2);
         P * rP = mixed_ ? reinterpret_cast<P *>(rP_.get()) : reinterpret_cast<P *>(r_.get());
         P * z = reinterpret_cast<P *>(z_.get());
-        byLanes(levels_[0].lanes, [&]<int LN>()
-                { amgInitKernel<P, LN, NCH><<<parts_, kBlock, 0, s>>>(a64_, b, x, r_.get(), rP, zeroGuess ? 1 : 0, st); });
+        const P * inv = levelMatrix<P>(0).invDiag;
+        const int c0End = fusedSweep() ? levels_[0].colorStart[1] : 0;
+        byRowLanes<NCH>(levels_[0].lanes, levels_[0].nnz / n_, [&]<int LN>()
+                        { amgInitKernel<P, LN, NCH><<<parts_, kBlock, 0, s>>>(a64_, b, x, r_.get(), rP, zeroGuess ? 1 : 0, st, z, inv, c0End); });
         amgInitFinalizeKernel<NCH><<<1, kBlock, 0, s>>>(st);
-        enqueueVcycle<P, NCH>(s, rP, z);
-        amgRhoKernel<P, NCH><<<parts_, kBlock, 0, s>>>(n_, r_.get(), z, st);
-        amgFinalizeKernel<NCH><<<1, kBlock, 0, s>>>(st, 1);
-        NSFEM_HIP(hipGetLastError());
+        enqueuePrecond<P, NCH>(s, rP, z, tol2, 1);
     }
 
     template <typename P, int NCH>
     void AmgPcg::enqueueIteration(hipStream_t s, double tol2)
     {
-        const AmgState st{scal_.get(), ints_.get(), active_.get(), partPq_.get(), partRr_.get(), partRho_.get(), partBb_.get(), parts_, tol2};
+        const AmgState st = state(tol2);
         P * rP = mixed_ ? reinterpret_cast<P *>(rP_.get()) : reinterpret_cast<P *>(r_.get());
         P * z = reinterpret_cast<P *>(z_.get());
-        byLanes(levels_[0].lanes, [&]<int LN>()
-                { amgDirectionKernel<P, LN, NCH><<<parts_, kBlock, 0, s>>>(a64_, z, p_.get(), q_.get(), st); });
-        amgUpdateKernel<P, NCH><<<parts_, kBlock, 0, s>>>(n_, p_.get(), q_.get(), xDevice_, r_.get(), rP, st);
-        enqueueVcycle<P, NCH>(s, rP, z);
-        amgRhoKernel<P, NCH><<<parts_, kBlock, 0, s>>>(n_, r_.get(), z, st);
-        amgFinalizeKernel<NCH><<<1, kBlock, 0, s>>>(st, 0);
-        NSFEM_HIP(hipGetLastError());
+        const P * inv = levelMatrix<P>(0).invDiag;
+        const int c0End = fusedSweep() ? levels_[0].colorStart[1] : 0;
+        byRowLanes<NCH>(levels_[0].lanes, levels_[0].nnz / n_, [&]<int LN>()
+                        { amgDirectionKernel<P, LN, NCH><<<parts_, kCgBlock<NCH>, 0, s>>>(a64_, z, p_.get(), q_.get(), st); });
+        amgUpdateKernel<P, NCH><<<parts_, kCgBlock<NCH>, 0, s>>>(n_, p_.get(), q_.get(), xDevice_, r_.get(), rP, st, z, inv, c0End);
+        enqueuePrecond<P, NCH>(s, rP, z, tol2, 0);
     }
 
     double AmgPcg::timeKernel(const std::string & which, int reps, double * bytesOut, double * launchesOut, double * x)
@@ -1164,7 +1707,7 @@ namespace nsfem
         fillInt(nch_, 1, active_.get(), s);
         fill(F64, 4L * nch_, 1.0, scal_.get(), s);
         fill(F64, static_cast<long>(parts_) * nch_, 1.0, partPq_.get(), s);
-        const AmgState st{scal_.get(), ints_.get(), active_.get(), partPq_.get(), partRr_.get(), partRho_.get(), partBb_.get(), parts_, tol2};
+        const AmgState st = state(tol2);
         if (x != xDevice_)
         {
             xDevice_ = x;
@@ -1174,19 +1717,21 @@ namespace nsfem
               {
                   P * rP = mixed_ ? reinterpret_cast<P *>(rP_.get()) : reinterpret_cast<P *>(r_.get());
                   P * z = reinterpret_cast<P *>(z_.get());
+                  const P * inv = levelMatrix<P>(0).invDiag;
+                  const int c0End = fusedSweep() ? levels_[0].colorStart[1] : 0;
                   if (which == "direction")
                   {
                       bytes = bDir;
                       launch = [=, this]()
                       {
-                          byLanes(levels_[0].lanes, [&]<int LN>()
-                                  { amgDirectionKernel<P, LN, NCH><<<parts_, kBlock, 0, s>>>(a64_, z, p_.get(), q_.get(), st); });
+                          byRowLanes<NCH>(levels_[0].lanes, levels_[0].nnz / n_, [&]<int LN>()
+                                  { amgDirectionKernel<P, LN, NCH><<<parts_, kCgBlock<NCH>, 0, s>>>(a64_, z, p_.get(), q_.get(), st); });
                       };
                   }
                   else if (which == "update")
                   {
                       bytes = bUpd;
-                      launch = [=, this]() { amgUpdateKernel<P, NCH><<<parts_, kBlock, 0, s>>>(n_, p_.get(), q_.get(), x, r_.get(), rP, st); };
+                      launch = [=, this]() { amgUpdateKernel<P, NCH><<<parts_, kCgBlock<NCH>, 0, s>>>(n_, p_.get(), q_.get(), x, r_.get(), rP, st, z, inv, c0End); };
                   }
                   else if (which == "rho")
                   {
@@ -1200,7 +1745,7 @@ namespace nsfem
                       bytes = bV;
                       hipGraph_t g = nullptr;
                       NSFEM_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-                      enqueueVcycle<P, NCH>(s, rP, z);
+                      enqueueVcycle<P, NCH>(s, rP, z, false, tol2);
                       NSFEM_HIP(hipStreamEndCapture(s, &g));
                       const hipError_t rc = hipGraphInstantiate(&vcycleExec, g, nullptr, nullptr, 0);
                       (void)hipGraphDestroy(g);

@@ -14,11 +14,12 @@
 // own CG scalars and stops on its own, the solve when all have stopped.
 //
 // Launches per iteration: the direction (p, q = A p and p.q partials), the
-// update (x, r, |r|^2 partials, the FP32 residual copy), the V-cycle (per
-// Gauss-Seidel level 2 x colours + 3, per Chebyshev level of degree k
-// 2 k + 2 (+1 on the finest, whose first iterate is not written by a
-// restriction), one dense product on the coarsest), the r.z partials and a
-// one-block finalize (rho, convergence).  Every kernel
+// update (x, r, |r|^2 partials, the FP32 residual copy, the first colour's start
+// of the forward sweep), the V-cycle (a Gauss-Seidel finest level 2 x colours
+// + 2, whose last backward colour forms the r.z partials, other Gauss-Seidel
+// levels 2 x colours + 3; a Chebyshev level of degree k 2 k + 2, one more and
+// the r.z partials' own on the finest; one dense product on the coarsest) and
+// a one-block finalize (rho, convergence).  Every kernel
 // returns at once after the solve has stopped, so whole iterations are
 // replayed from one captured graph and polled one iteration behind.
 #pragma once
@@ -33,6 +34,20 @@
 
 namespace nsfem
 {
+    // Device scalars and partial sums of one solve.
+    struct AmgState
+    {
+        double * scal; // per channel, blocks of NCH: rho, rho of the iteration before, |b|^2, |r|^2
+        int * ints;    // stop (0 running, 1 converged, 2 non-finite or breakdown), iterations, zero right-hand sides
+        int * active;  // per channel
+        double * partPq;
+        double * partRr;
+        double * partRho;
+        double * partBb;
+        int parts;
+        double tol2;
+    };
+
     class AmgPcg
     {
     public:
@@ -123,8 +138,17 @@ namespace nsfem
 
         template <typename T>
         McgsMatrix<T> levelMatrix(int l) const;
+        AmgState state(double tol2);
+        // The finest level's Gauss-Seidel sweeps start with the residual's
+        // kernel and end with r.z (not with a Chebyshev finest level or a
+        // one-level hierarchy).
+        bool fusedSweep() const { return numLevels() > 1 && levels_[0].chebDegree == 0; }
+        // fused: without the finest level's first forward colour, and with
+        // the partial sums of r.z in its last backward colour
         template <typename T, int NCH>
-        void enqueueVcycle(hipStream_t s, const T * b0, T * x0);
+        void enqueueVcycle(hipStream_t s, const T * b0, T * x0, bool fused, double tol2);
+        template <typename P, int NCH>
+        void enqueuePrecond(hipStream_t s, const P * rP, P * z, double tol2, int init);
         template <typename P, int NCH>
         void enqueueInit(hipStream_t s, const double * b, double * x, bool zeroGuess, double tol2);
         template <typename P, int NCH>
@@ -140,7 +164,7 @@ namespace nsfem
         McgsMatrix<double> a64_{};
         McgsMatrix<float> a32_{};
         std::vector<Level> levels_;
-        int coarseN_ = 0;
+        int coarseN_ = 0, coarseLd_ = 0;
         DeviceArray<double> coarse64_;
         DeviceArray<float> coarse32_;
         double complexity_ = 0, setupSeconds_ = 0;

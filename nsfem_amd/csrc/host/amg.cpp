@@ -266,10 +266,10 @@ namespace nsfem
             return agg;
         }
 
-        // Dense inverse of an SPD matrix (Cholesky, then L^-T L^-1); singular:
-        // of A + s 1 1^T, s = mean diagonal / n (A positive semidefinite with
-        // the constants as its null space).
-        std::vector<double> denseInverse(const CsrD & a, bool singular)
+        // The coarsest operator as a dense matrix; singular: A + s 1 1^T, s = mean
+        // diagonal / n (A positive semidefinite with the constants as its null
+        // space).
+        std::vector<double> denseMatrix(const CsrD & a, bool singular)
         {
             const int n = a.rows;
             std::vector<double> m(static_cast<size_t>(n) * n, 0.0);
@@ -293,6 +293,14 @@ namespace nsfem
                     v += shift;
                 }
             }
+            return m;
+        }
+
+        // Its inverse (Cholesky, then L^-T L^-1).
+        std::vector<double> denseInverse(const CsrD & a, bool singular)
+        {
+            const int n = a.rows;
+            std::vector<double> m = denseMatrix(a, singular);
             // lower Cholesky factor in place
             for (int j = 0; j < n; j++)
             {
@@ -400,20 +408,31 @@ namespace nsfem
         }
         double nnz0 = stripped.nnz() + n0, nnzAll = nnz0;
         double theta = opt.theta;
+        auto finish = [&](const CsrD & A)
+        {
+            if (opt.invertCoarse)
+            {
+                h.coarseInverse = denseInverse(A, h.singular);
+            }
+            else
+            {
+                h.coarseMatrix = denseMatrix(A, h.singular);
+            }
+        };
         for (;;)
         {
             AmgLevel & L = h.levels.back();
             const CsrD A = assemble(L);
             if (L.n <= opt.maxCoarse || static_cast<int>(h.levels.size()) >= opt.maxLevels)
             {
-                h.coarseInverse = denseInverse(A, h.singular);
+                finish(A);
                 break;
             }
             int nc = 0;
             const std::vector<int> agg = aggregate(A, L.diag, theta, nc);
             if (nc >= L.n || nc < 1)
             {
-                h.coarseInverse = denseInverse(A, h.singular); // no coarsening left
+                finish(A); // no coarsening left
                 break;
             }
             // smoothed prolongation P = (I - omega D^-1 A) P_tent

@@ -31,6 +31,9 @@ namespace nsfem
         int maxCoarse = 512;     // the coarsest level has at most this many rows
         int maxLevels = 12;
         double omegaScale = 4.0 / 3.0;
+        // false: leave the coarsest operator's inverse to the caller
+        // (coarseMatrix instead of coarseInverse)
+        bool invertCoarse = true;
     };
 
     struct AmgLevel
@@ -56,6 +59,7 @@ namespace nsfem
     {
         std::vector<AmgLevel> levels;
         std::vector<double> coarseInverse; // coarsest n x n, row-major
+        std::vector<double> coarseMatrix;  // the matrix to invert (invertCoarse = false)
         double operatorComplexity = 0;     // sum of nnz over the levels / nnz of the finest
         // Zero row sums on the finest level (a pure-Neumann Laplacian): the
         // constants span the null space on every level (P maps constants to

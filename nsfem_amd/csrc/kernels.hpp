@@ -1333,10 +1333,10 @@ namespace nsfem
     // Sum over count partial slots of channel threadIdx.x % NCH (slot i,
     // channel c at parts[i*NCH + c]); the total of channel c is returned in
     // thread c (c < NCH).  Same order in every block.
-    template <int NCH>
+    template <int NCH, int BLOCK = kBlock>
     __device__ __forceinline__ double channelPartialSum(const double * __restrict__ parts, int count, double * sm)
     {
-        constexpr int G = kBlock / NCH; // threads per channel
+        constexpr int G = BLOCK / NCH; // threads per channel
         const int c = static_cast<int>(threadIdx.x) % NCH;
         double acc = 0;
 #pragma unroll 4
@@ -1344,7 +1344,7 @@ namespace nsfem
         {
             acc += parts[static_cast<size_t>(i) * NCH + c];
         }
-        return channelBlockSum<NCH>(acc, sm);
+        return channelBlockSum<NCH, BLOCK / 64>(acc, sm);
     }
 
     // Fused reductions, first half: the flags, the system's per-channel state
