@@ -129,7 +129,8 @@ namespace nsfem
     // Plain CSR products: y = alpha * A x (+ beta y), NCH planar channels.
     // rowIds != nullptr: output row i is A's row rowIds[i] (fused gather).
     // ------------------------------------------------------------------
-    template <typename T, int LANES, int NCH>
+    // U: entries per lane and step (0: from the lanes, as below).
+    template <typename T, int LANES, int NCH, int UNROLL = 0>
     __global__ void __launch_bounds__(kBlock) csrMulKernel(int rows, const int * __restrict__ rowStart,
                                                             const int * __restrict__ column, const T * __restrict__ values,
                                                             const T * __restrict__ x, long ldx, T * __restrict__ y, long ldy,
@@ -155,7 +156,7 @@ namespace nsfem
             // of 8 or more take one entry per step: their lanes see about one
             // entry of a row each, and the reloads measured slower (P2 rows,
             // 8 lanes: 155 -> 171 us at 2M rows).
-            constexpr int U = LANES <= 2 ? 4 : (LANES <= 4 ? 2 : 1);
+            constexpr int U = UNROLL > 0 ? UNROLL : (LANES <= 2 ? 4 : (LANES <= 4 ? 2 : 1));
             for (int j = rowStart[src] + lane; j < j1; j += U * LANES)
             {
                 T v[U];
@@ -1373,9 +1374,11 @@ namespace nsfem
 #pragma unroll
         for (int k = 0; k < PRE; k++)
         {
+            // unconditional (slot 0 past the end, dropped below): loads under a
+            // condition wait for one another
             const int i = i0 + k * G;
-            f.rho[k] = i < sl.rhoParts ? pr[static_cast<size_t>(i) * NCH + c] : 0.0;
-            f.rr[k] = i < sl.updParts ? pu[static_cast<size_t>(i) * NCH + c] : 0.0;
+            f.rho[k] = pr[static_cast<size_t>(i < sl.rhoParts ? i : 0) * NCH + c];
+            f.rr[k] = pu[static_cast<size_t>(i < sl.updParts ? i : 0) * NCH + c];
         }
     }
 
@@ -1400,16 +1403,19 @@ namespace nsfem
 #pragma unroll
         for (int k = 0; k < PRE; k++)
         {
-            rho += f.rho[k];
-            rr += f.rr[k];
+            const int i = t / NCH + k * G;
+            rho += i < sl.rhoParts ? f.rho[k] : 0.0;
+            rr += i < sl.updParts ? f.rr[k] : 0.0;
         }
         // beyond the preloaded slots (more than PRE * G partials)
         const double * pr = st.partials + static_cast<size_t>(sl.base) * NCH;
         const double * pu = st.partials2 + static_cast<size_t>(sl.base) * NCH;
+#pragma unroll 4
         for (int i = t / NCH + PRE * G; i < sl.rhoParts; i += G)
         {
             rho += pr[static_cast<size_t>(i) * NCH + c];
         }
+#pragma unroll 4
         for (int i = t / NCH + PRE * G; i < sl.updParts; i += G)
         {
             rr += pu[static_cast<size_t>(i) * NCH + c];
@@ -2022,13 +2028,13 @@ namespace nsfem
     // same alpha = rho / p.q) while its first elements' operands are already
     // loading, with rho and activity as the direction kernel decided them;
     // block 0 makes those decisions the solve state for the kernels that follow.
-    template <typename T, typename P, int NCH>
-    __global__ void __launch_bounds__(kBlock) pcgUpdateKernel(int n, BlockMap bm, SolveState st, const T * __restrict__ p,
+    template <typename T, typename P, int NCH, int BLOCK = kBlock>
+    __global__ void __launch_bounds__(BLOCK) pcgUpdateKernel(int n, BlockMap bm, SolveState st, const T * __restrict__ p,
                                                               const T * __restrict__ q, T * __restrict__ x, T * r, P * rP,
                                                               P * __restrict__ z, const P * __restrict__ invDiagP, int color0End,
                                                               int fused, int dirParts)
     {
-        __shared__ double sm[NCH * kWaves];
+        __shared__ double sm[NCH * (BLOCK / 64)];
         __shared__ double shAlpha[NCH];
         __shared__ int shAct[NCH];
         const int lb = logicalBlock(blockIdx.x, gridDim.x);
@@ -2036,8 +2042,8 @@ namespace nsfem
         const int4 range = blockRange(bm, lb);
         const int s = range.z;
         // flat over the block's interleaved elements, one per thread: the
-        // stride (kBlock) is a multiple of NCH, so a thread keeps one channel
-        static_assert(kBlock % NCH == 0, "channels must divide the block");
+        // stride (BLOCK) is a multiple of NCH, so a thread keeps one channel
+        static_assert(BLOCK % NCH == 0, "channels must divide the block");
         const int c = static_cast<int>(threadIdx.x) % NCH;
         const long i0 = static_cast<long>(range.x) * NCH + threadIdx.x;
         const long end = static_cast<long>(range.y) * NCH;
@@ -2079,7 +2085,7 @@ namespace nsfem
                 }
             }
             const FusedSlice sl = fusedSlice(bm, range, lb, dirParts, dirParts);
-            const double pq = channelPartialSum<NCH>(st.partials3 + static_cast<size_t>(sl.base) * NCH, sl.rhoParts, sm);
+            const double pq = channelPartialSum<NCH, BLOCK>(st.partials3 + static_cast<size_t>(sl.base) * NCH, sl.rhoParts, sm);
             // block 0 makes the direction kernel's decisions (every system)
             // the solve state, also when they stop the solve; no block of
             // this launch reads what it writes: the blocks test their own
@@ -2088,7 +2094,7 @@ namespace nsfem
             {
                 const int K = bm.numSystems * NCH;
                 int any = 0;
-                for (int k = t; k < K; k += kBlock)
+                for (int k = t; k < K; k += BLOCK)
                 {
                     const int a = st.activeNext[k];
                     st.active[k] = a;
@@ -2173,7 +2179,7 @@ namespace nsfem
             {
                 finish(i0, row0, r0, x0, p0, q0, d0);
             }
-            for (long i = i0 + kBlock; i < end; i += kBlock)
+            for (long i = i0 + BLOCK; i < end; i += BLOCK)
             {
                 const int row = static_cast<int>(i / NCH);
                 const T ri = r[i];
@@ -2190,7 +2196,7 @@ namespace nsfem
         }
         if constexpr (kWide<NCH>)
         {
-            const double total = channelBlockSum<NCH>(sum, sm);
+            const double total = channelBlockSum<NCH, BLOCK / 64>(sum, sm);
             storeChannelPartial<NCH, NCH>(total, st.partials2, range.w, 0);
         }
         else
@@ -2201,7 +2207,7 @@ namespace nsfem
             {
                 part[cc] = cc == c ? sum : 0.0;
             }
-            blockSum<NCH>(part, sm);
+            blockSum<NCH, BLOCK / 64>(part, sm);
             storePartial<NCH>(part, st.partials2, range.w);
         }
     }

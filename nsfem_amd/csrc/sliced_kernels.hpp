@@ -336,4 +336,249 @@ namespace nsfem
         blockSum<NCH, W>(part, sm);
         storePartial<NCH>(part, st.partials, range.w);
     }
+
+    // ------------------------------------------------------------------
+    // Four to 32 channels on the same rows in CSR form: one lane per channel
+    // (a gathered column is NCH contiguous values), workgroups of 1,024
+    // threads.  bm.blocks holds ranges of rows.
+    //
+    // Every workgroup of the next kernel re-sums this one's partial sums, NCH
+    // for each workgroup, so few and large ones: one on every CU, two where
+    // the vectors are so long that the sums do not count.  P2 mass matrix, 16
+    // channels, mixed: an iteration at 40k pressure nodes 92 us (128 / 512
+    // workgroups 153 / 96), at 500k 1,149 us with 512 (1,372 with 256).  The
+    // kernels before, 64 rows to a workgroup in colour order, took 200 and
+    // 2,511 us: direction 82 -> 35, each factor launch 47 -> 18 us at 40k.
+    // ------------------------------------------------------------------
+    constexpr int kWideBlock = 1024;
+    constexpr int kWideWaves = kWideBlock / 64;
+    constexpr int kWideGroups = 256, kWideGroupsLong = 512;
+    constexpr long kWideLong = 8L << 20; // values of a vector from which on two pay
+
+    // The product of the row whose entries are [j0, j1) for the lane's channel,
+    // NCH lanes a row.  The lanes load NCH entries at once and pass them around:
+    // loaded where they are used, values and columns are two of three vector
+    // memory instructions, each as long as a gather, and those bound the kernel
+    // (40k pressure nodes x 16
+    // channels: direction 41 -> 35 us in mixed precision, 51 -> 38 in FP64).
+    // Every lane of the wavefront takes part (the bounds of its loops are
+    // the wavefront's).
+    template <int U, int NCH, typename V, typename X>
+    __device__ __forceinline__ V channelRowDot(int j0, int j1, const int * __restrict__ column, const V * __restrict__ values,
+                                               const X * __restrict__ x)
+    {
+        const int lane = static_cast<int>(threadIdx.x) & 63;
+        const int c = lane % NCH, group = lane - c;
+        constexpr int K = U < NCH ? U : NCH;
+        V acc = V(0);
+        for (int jb = j0; __any(jb < j1); jb += NCH)
+        {
+            const int count = j1 - jb;
+            const int e = c < count ? jb + c : 0; // (entry 0 exists; its term is dropped)
+            const V v = values[e];
+            const int col = column[e];
+            for (int u = 0; u < NCH && __any(u < count); u += K)
+            {
+                X xv[K];
+#pragma unroll
+                for (int k = 0; k < K; k++)
+                {
+                    xv[k] = x[static_cast<long>(__shfl(col, group + u + k, 64)) * NCH + c];
+                }
+#pragma unroll
+                for (int k = 0; k < K; k++)
+                {
+                    const V vk = __shfl(v, group + u + k, 64);
+                    acc = u + k < count ? fmaT(vk, static_cast<V>(xv[k]), acc) : acc;
+                }
+            }
+        }
+        return acc;
+    }
+
+    // Rows range.x + t / NCH, + kWideBlock / NCH, ...: own(row) loads the row's
+    // operands, part(row, acc) takes its product.  The next row's bounds load
+    // with the current row's entries; U entries go out together.  begin() runs
+    // once, behind the first row's loads (every thread; false ends the kernel).
+    template <int U, int NCH, typename V, typename X, typename Begin, typename Own, typename Part>
+    __device__ __forceinline__ bool wideRows(const int * __restrict__ start, const int * __restrict__ end, const int * __restrict__ column,
+                                             const V * __restrict__ values, int4 range, const X * __restrict__ x, Begin begin, Own own,
+                                             Part part)
+    {
+        constexpr int step = kWideBlock / NCH;
+        const int c = static_cast<int>(threadIdx.x) % NCH;
+        int row = range.x + static_cast<int>(threadIdx.x) / NCH;
+        int rs = row < range.y ? row : range.x;
+        int j0 = start[rs], j1 = end[rs];
+        if (!begin())
+        {
+            return false;
+        }
+        for (int base = range.x; base < range.y; base += step, row += step)
+        {
+            const bool valid = row < range.y;
+            own(rs);
+            const int next = row + step < range.y ? row + step : range.x;
+            const int n0 = start[next], n1 = end[next];
+            const V acc = channelRowDot<U, NCH>(j0, valid ? j1 : j0, column, values, x);
+            if (valid)
+            {
+                part(row, acc);
+            }
+            rs = next;
+            j0 = n0;
+            j1 = n1;
+        }
+        return true;
+    }
+
+    template <typename T, typename P, int NCH>
+    __global__ void __launch_bounds__(kWideBlock, 8) wideDirectionKernel(McgsMatrix<T> A, BlockMap bm, SolveState st,
+                                                                         const P * __restrict__ z, T * __restrict__ p, T * __restrict__ q)
+    {
+        constexpr int PRE = 4; // 256 workgroups' partial sums of 16 channels
+        __shared__ double sm[2 * NCH * kWideWaves];
+        __shared__ double shBeta[NCH];
+        __shared__ int shAct[NCH];
+        const int lb = logicalBlock(blockIdx.x, gridDim.x);
+        const int4 range = bm.blocks[lb];
+        if (st.flags[0])
+        {
+            return;
+        }
+        const FusedSlice sl = fusedSlice(bm, range, lb, 0, 0);
+        const bool first = st.flags[1] != 0;
+        FusedRhoLoads<NCH, kWideBlock, PRE> fl;
+        fusedRhoLoad<NCH, kWideBlock, PRE>(st, sl, fl);
+        const int c = static_cast<int>(threadIdx.x) % NCH;
+        T beta = T(0), dg = T(0), pr = T(0), qr = T(0);
+        P zr = P(0);
+        double sum = 0;
+        const bool go = wideRows<4, NCH>(
+            A.rowStart, A.rowStart + 1, A.column, A.values, range, z,
+            [&]()
+            {
+                const bool any = fusedRhoFinish<NCH, kWideBlock, PRE>(st, fl, sl, sm, shBeta, shAct);
+                beta = static_cast<T>(shBeta[c]);
+                return any;
+            },
+            [&](int row)
+            {
+                const long i = static_cast<long>(row) * NCH + c;
+                dg = A.diag[row];
+                zr = z[i];
+                pr = p[i];
+                qr = q[i];
+            },
+            [&](int row, T acc)
+            {
+                const long i = static_cast<long>(row) * NCH + c;
+                const T zi = static_cast<T>(zr);
+                const T az = fmaT(dg, zi, acc);
+                const T pi = first ? zi : fmaT(beta, pr, zi);
+                const T qi = first ? az : fmaT(beta, qr, az);
+                p[i] = pi;
+                q[i] = qi;
+                sum = fma(static_cast<double>(pi), static_cast<double>(qi), sum);
+            });
+        if (!go)
+        {
+            return;
+        }
+        const double total = channelBlockSum<NCH, kWideWaves>(sum, sm);
+        storeChannelPartial<NCH, NCH>(total, st.partials3, range.w, 0);
+    }
+
+    template <typename T, typename P, int NCH>
+    __global__ void __launch_bounds__(kWideBlock, 8) wideInitKernel(McgsMatrix<T> A, BlockMap bm, SolveState st, const T * __restrict__ b,
+                                                                    const T * __restrict__ x, T * r, P * rP)
+    {
+        __shared__ double sm[2 * NCH * kWideWaves];
+        const int4 range = bm.blocks[logicalBlock(blockIdx.x, gridDim.x)];
+        const int c = static_cast<int>(threadIdx.x) % NCH;
+        T dg = T(0), xr = T(0), br = T(0);
+        double bb = 0, rr = 0;
+        wideRows<4, NCH>(
+            A.rowStart, A.rowStart + 1, A.column, A.values, range, x, []() { return true; },
+            [&](int row)
+            {
+                const long i = static_cast<long>(row) * NCH + c;
+                dg = A.diag[row];
+                xr = x[i];
+                br = b[i];
+            },
+            [&](int row, T acc)
+            {
+                const long i = static_cast<long>(row) * NCH + c;
+                const T ri = br - fmaT(dg, xr, acc);
+                r[i] = ri;
+                if constexpr (!std::is_same_v<T, P>)
+                {
+                    rP[i] = static_cast<P>(ri);
+                }
+                bb = fma(static_cast<double>(br), static_cast<double>(br), bb);
+                rr = fma(static_cast<double>(ri), static_cast<double>(ri), rr);
+            });
+        channelBlockSum2<NCH, kWideWaves>(bb, rr, sm);
+        storeChannelPartial<NCH, 2 * NCH>(bb, st.partials, range.w, 0);
+        storeChannelPartial<NCH, 2 * NCH>(rr, st.partials, range.w, NCH);
+    }
+
+    template <typename P, int NCH>
+    __global__ void __launch_bounds__(kWideBlock, 8) wideLowerKernel(McgsMatrix<P> G, BlockMap bm, SolveState st, const P * __restrict__ r,
+                                                                     P * __restrict__ t)
+    {
+        const int4 range = bm.blocks[logicalBlock(blockIdx.x, gridDim.x)];
+        if (st.flags[0] || !systemActive<NCH>(st, range.z))
+        {
+            return;
+        }
+        const int c = static_cast<int>(threadIdx.x) % NCH;
+        P dg = P(0), rv = P(0);
+        wideRows<8, NCH>(
+            G.rowStart, G.rowSplit, G.column, G.values, range, r, []() { return true; },
+            [&](int row)
+            {
+                dg = G.diag[row];
+                rv = r[static_cast<long>(row) * NCH + c];
+            },
+            [&](int row, P acc) { t[static_cast<long>(row) * NCH + c] = fmaT(dg, rv, acc); });
+    }
+
+    template <typename P, typename T, int NCH>
+    __global__ void __launch_bounds__(kWideBlock, 8) wideUpperKernel(McgsMatrix<P> G, BlockMap bm, SolveState st, const P * __restrict__ t,
+                                                                     P * __restrict__ z, const T * __restrict__ r)
+    {
+        __shared__ double sm[NCH * kWideWaves];
+        const int4 range = bm.blocks[logicalBlock(blockIdx.x, gridDim.x)];
+        if (st.flags[0])
+        {
+            return;
+        }
+        const int c = static_cast<int>(threadIdx.x) % NCH;
+        double sum = 0;
+        if (systemActive<NCH>(st, range.z))
+        {
+            P dg = P(0), tv = P(0);
+            T rv = T(0);
+            wideRows<8, NCH>(
+                G.rowSplit, G.rowStart + 1, G.column, G.values, range, t, []() { return true; },
+                [&](int row)
+                {
+                    const long i = static_cast<long>(row) * NCH + c;
+                    dg = G.diag[row];
+                    tv = t[i];
+                    rv = r[i];
+                },
+                [&](int row, P acc)
+                {
+                    const long i = static_cast<long>(row) * NCH + c;
+                    const P zi = fmaT(dg, tv, acc);
+                    z[i] = zi;
+                    sum = fma(static_cast<double>(rv), static_cast<double>(zi), sum);
+                });
+        }
+        const double total = channelBlockSum<NCH, kWideWaves>(sum, sm);
+        storeChannelPartial<NCH, NCH>(total, st.partials, range.w, 0);
+    }
 } // namespace nsfem

@@ -878,7 +878,7 @@ namespace nsfem
             nbDir_ = nbUpd_ = nbRho_ = nbPre_ = numBlocks_;
             color0BlocksRho_ = color0Blocks_;
         }
-        if (sliced())
+        if (sliced() || wideLocal())
         {
             setupSliceMaps();
             maxBlocks = std::max(maxBlocks, nbDir_);
@@ -1004,6 +1004,11 @@ namespace nsfem
             loc_.g32.upload(to32(gv));
             loc_.gDiag32.upload(to32(gd));
         }
+        loc_.systemSlice.assign(1, 0);
+        for (const RowChunk & ch : loc_.chunks)
+        {
+            loc_.systemSlice.push_back(loc_.systemSlice.back() + (ch.end - ch.begin + 63) / 64);
+        }
         if (opt_.numCh > 2)
         {
             return;
@@ -1015,7 +1020,6 @@ namespace nsfem
             std::vector<int4> table;
             std::vector<int> sc;
             std::vector<double> sv;
-            loc_.systemSlice.assign(1, 0);
             for (const RowChunk & ch : loc_.chunks)
             {
                 for (int r0 = ch.begin; r0 < ch.end; r0 += 64)
@@ -1046,7 +1050,6 @@ namespace nsfem
                         }
                     }
                 }
-                loc_.systemSlice.push_back(static_cast<int>(table.size()));
             }
             if (sc.empty())
             {
@@ -1071,7 +1074,7 @@ namespace nsfem
 
     void McgsSolver::setupSliceMaps()
     {
-        // Each system's slices go to its share of kSliceGroups workgroups; every
+        // Each system's slices go to its share of the workgroups; every
         // kernel of the iteration uses the same workgroups, so all partial
         // sums share their slots.
         const int total = loc_.systemSlice.back();
@@ -1080,7 +1083,11 @@ namespace nsfem
         // 16.8 / 18.8, 690 slices 18.8 / 17.8 / 19.1, 1,890 slices 30.5 / 26.1
         // / 25.7, 7,550 slices 65.7 / 51.8 / 49.4).
         loc_.waves = total > 1024 ? 8 : (total > 256 ? 4 : 2);
-        const int per = std::max(loc_.waves, (total + kSliceGroups - 1) / kSliceGroups); // slices per workgroup
+        // slices per workgroup (wide tiles: 1,024 threads are NCH lanes on 1,024 / NCH rows)
+        const int least = wideLocal() ? std::max(1, kWideWaves / opt_.numCh) : loc_.waves;
+        const bool longVectors = static_cast<long>(n_) * opt_.numCh > kWideLong;
+        const int groups = wideLocal() ? (longVectors ? kWideGroupsLong : kWideGroups) : kSliceGroups;
+        const int per = std::max(least, (total + groups - 1) / groups);
         std::vector<int> start(1, 0);
         for (int s = 0; s < numSystems_; s++)
         {
@@ -1142,6 +1149,16 @@ namespace nsfem
                           nch == 1 ? go.template operator()<1>() : go.template operator()<2>();
                       });
         }
+        else if (wideLocal() && !zeroGuess)
+        {
+            dispatchC(nch, [&]<int C>()
+                      {
+                          if constexpr (kWide<C>)
+                          {
+                              wideInitKernel<T, P, C><<<nbDir_, kWideBlock, 0, s>>>(v.A, loc_.rows, st, v.b, v.x, v.r, v.rP);
+                          }
+                      });
+        }
         else
         {
             // r = b - A x is the direction kernel's product: its map and lanes
@@ -1170,10 +1187,41 @@ namespace nsfem
                       });
             return;
         }
+        if (wideLocal())
+        {
+            dispatchC(nch, [&]<int C>()
+                      {
+                          if constexpr (kWide<C>)
+                          {
+                              wideDirectionKernel<T, P, C><<<nbDir_, kWideBlock, 0, s>>>(v.A, loc_.rows, st, v.z, v.p, v.q);
+                          }
+                      });
+            return;
+        }
         dispatchLC(directionLanes(), nch, [&]<int L, int C>()
                    {
                        pcgDirectionKernel<T, P, L, C><<<nbDir_, kBlock, 0, s>>>(v.A, bmDir_, st, v.z, v.p, v.q, fz, rhoParts(), nbUpd_);
                    });
+    }
+
+    template <typename T, typename P>
+    void McgsSolver::launchUpdate(hipStream_t s, const PcgOperands<T, P> & v, SolveState st)
+    {
+        const int fz = fused() ? 1 : 0;
+        dispatchC(opt_.numCh, [&]<int C>()
+                  {
+                      if constexpr (kWide<C>)
+                      {
+                          if (wideLocal())
+                          {
+                              pcgUpdateKernel<T, P, C, kWideBlock><<<nbUpd_, kWideBlock, 0, s>>>(
+                                  n_, bmUpd_, st, v.p, v.q, v.x, v.r, v.rP, v.z, v.M.invDiag, zColour0End(), fz, nbDir_);
+                              return;
+                          }
+                      }
+                      pcgUpdateKernel<T, P, C><<<nbUpd_, kBlock, 0, s>>>(n_, bmUpd_, st, v.p, v.q, v.x, v.r, v.rP, v.z, v.M.invDiag,
+                                                                        zColour0End(), fz, nbDir_);
+                  });
     }
 
     template <typename T, typename P>
@@ -1191,6 +1239,18 @@ namespace nsfem
                                                                                      v.z, v.r);
                           };
                           nch == 1 ? go.template operator()<1>() : go.template operator()<2>();
+                      });
+            return;
+        }
+        if (wideLocal())
+        {
+            dispatchC(nch, [&]<int C>()
+                      {
+                          if constexpr (kWide<C>)
+                          {
+                              wideLowerKernel<P, C><<<nbPre_, kWideBlock, 0, s>>>(v.G, loc_.rows, st, v.rP, v.t);
+                              wideUpperKernel<P, T, C><<<nbPre_, kWideBlock, 0, s>>>(v.G, loc_.rows, st, v.t, v.z, v.r);
+                          }
                       });
             return;
         }
@@ -1630,11 +1690,7 @@ namespace nsfem
         }
         else
         {
-            dispatchC(nch, [&]<int C>()
-                      {
-                          pcgUpdateKernel<T, P, C><<<nbUpd_, kBlock, 0, s>>>(n_, bmUpd_, st, v.p, v.q, v.x, v.r, v.rP, v.z, v.M.invDiag,
-                                                                            zColour0End(), fz, nbDir_);
-                      });
+            launchUpdate<T, P>(s, v, st);
         }
         // the update's convergence test is finished together with rho
         launchPrecond<T, P>(s, v, st, totals, true);
@@ -2638,14 +2694,7 @@ namespace nsfem
                 }
                 else
                 {
-                    launch = [=, this]()
-                    {
-                        dispatchC(nch, [&]<int C>()
-                                  {
-                                      pcgUpdateKernel<T, P, C><<<nbUpd_, kBlock, 0, s>>>(n_, bmUpd_, st, v.p, v.q, v.x, v.r, v.rP,
-                                                                                        v.z, v.M.invDiag, zColour0End(), fz, nbDir_);
-                                  });
-                    };
+                    launch = [=, this]() { launchUpdate<T, P>(s, v, st); };
                 }
             }
             else if (which == "finalize")

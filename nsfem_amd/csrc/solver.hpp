@@ -325,6 +325,8 @@ namespace nsfem
         // ... and, with fused reductions on one or two channels, its products
         // on slices of 64 rows (sliced_kernels.hpp)
         bool sliced() const { return local() && fused() && opt_.numCh <= 2; }
+        // ... and on more channels in workgroups of 1,024 threads (wideRows)
+        bool wideLocal() const { return local() && fused() && opt_.numCh > 2; }
         void buildLocal(const std::vector<int> & rowStart, const std::vector<int> & rowSplit, const std::vector<int> & column,
                         const std::vector<double> & values, const std::vector<double> & diag, const std::vector<double> & g,
                         const std::vector<double> & gDiag);
@@ -335,6 +337,8 @@ namespace nsfem
         void launchInit(hipStream_t s, const PcgOperands<T, P> & v, SolveState st, bool zeroGuess, const int * gate, double * totals);
         template <typename T, typename P>
         void launchDirection(hipStream_t s, const PcgOperands<T, P> & v, SolveState st);
+        template <typename T, typename P>
+        void launchUpdate(hipStream_t s, const PcgOperands<T, P> & v, SolveState st);
         template <typename T, typename P>
         void launchApproximateInverse(hipStream_t s, const PcgOperands<T, P> & v, SolveState st);
         void runMixedRestart(hipStream_t s);

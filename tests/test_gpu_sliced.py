@@ -1,6 +1,7 @@
-"""PCG with the approximate inverse on sliced rows in locality order against
-the general kernels (two finalize launches per iteration, which walk the same
-rows in CSR form): edges of the slices, empty and long rows, several systems."""
+"""PCG with the approximate inverse on sliced rows in locality order (from four
+channels on in CSR form, one lane per channel) against the general kernels
+(two finalize launches per iteration): edges of the slices, empty and long
+rows, several systems."""
 
 import numpy as np
 import pytest
@@ -43,11 +44,13 @@ def _run(name, nch, mats, b, x0, fused, dtype, target):
 # slices; a window of 1,024 rows is sorted together
 @pytest.mark.parametrize("sizes", [[1], [63], [64], [65], [1023], [1025], [257 * 64 + 1], [1025 * 64 + 5], [40, 1, 700, 64, 130]])
 @pytest.mark.parametrize("name,nch,dtype", [("pcg", 1, np.float64), ("pcg", 2, np.float64), ("pcg_mixed", 2, np.float64),
-                                            ("pcg_mixed", 1, np.float64), ("pcg", 2, np.float32)])
+                                            ("pcg_mixed", 1, np.float64), ("pcg", 2, np.float32), ("pcg", 4, np.float64),
+                                            ("pcg_mixed", 8, np.float64), ("pcg_mixed", 16, np.float64), ("pcg", 16, np.float32),
+                                            ("pcg", 32, np.float64)])
 @pytest.mark.parametrize("kind", ["sparse", "long", "diagonal"])
 def test_sliced_solves_equal_the_general_kernels(sizes, name, nch, dtype, kind):
-    if kind != "sparse" and max(sizes) > 20_000:
-        pytest.skip("the long-row pattern is built densely")
+    if (kind != "sparse" or nch > 2) and max(sizes) > 20_000:
+        pytest.skip("one or two channels and one pattern reach the largest sizes")
     mats = [_spd(n, 100 + n, kind) for n in sizes]
     n = sum(sizes)
     rng = np.random.default_rng(7)
