@@ -29,6 +29,10 @@ namespace nsfem
         template <typename T, int L, int NCH, typename V>
         __device__ __forceinline__ T rowDotChannels(const McgsMatrix<T> & A, int j0, int j1, const V * __restrict__ v)
         {
+            if constexpr (L == NCH)
+            {
+                return channelRowDot<8, NCH>(j0, j1, A.column, A.values, v);
+            }
             constexpr int E = L / NCH, U = 4;
             const int lane = static_cast<int>(threadIdx.x) % L;
             const int c = lane % NCH, g = lane / NCH;
@@ -1069,18 +1073,25 @@ namespace nsfem
             }
         }
 
-        // f<L>(): lanes per row; four channels or more take NCH lanes per
-        // group and as many groups as keep a mean row to one or two rounds
+        // f<L>(): lanes per row.  Four and eight channels take as many groups of
+        // NCH lanes as keep a mean row to one or two rounds of loads; sixteen
+        // take one group, which passes its entries around (us an iteration,
+        // FP32 V-cycle, one group / more: 100k x 16 136 / 157, 40k x 8 86 / 84,
+        // 200k x 4 128 / 118).
         template <int NCH, typename F>
         void byRowLanes(int lanes, double meanRow, F && f)
         {
-            if constexpr (kChannelLanes<NCH>)
+            if constexpr (NCH >= 16)
+            {
+                f.template operator()<NCH>();
+            }
+            else if constexpr (kChannelLanes<NCH>)
             {
                 if (meanRow < 4)
                 {
                     f.template operator()<NCH>();
                 }
-                else if (meanRow < 10 || 4 * NCH > 64)
+                else if (meanRow < 10)
                 {
                     f.template operator()<2 * NCH>();
                 }
@@ -1088,6 +1099,20 @@ namespace nsfem
                 {
                     f.template operator()<4 * NCH>();
                 }
+            }
+            else
+            {
+                byLanes(lanes, f);
+            }
+        }
+        // The FP64 products around the V-cycle: one group on any channel count
+        // (direction, 200k x 4 17.1 -> 14.7 us, 100k x 16 29.1 -> 18.4).
+        template <int NCH, typename F>
+        void byProductLanes(int lanes, F && f)
+        {
+            if constexpr (kChannelLanes<NCH>)
+            {
+                f.template operator()<NCH>();
             }
             else
             {
@@ -1638,7 +1663,7 @@ namespace nsfem
         P * z = reinterpret_cast<P *>(z_.get());
         const P * inv = levelMatrix<P>(0).invDiag;
         const int c0End = fusedSweep() ? levels_[0].colorStart[1] : 0;
-        byRowLanes<NCH>(levels_[0].lanes, levels_[0].nnz / n_, [&]<int LN>()
+        byProductLanes<NCH>(levels_[0].lanes, [&]<int LN>()
                         { amgInitKernel<P, LN, NCH><<<parts_, kBlock, 0, s>>>(a64_, b, x, r_.get(), rP, zeroGuess ? 1 : 0, st, z, inv, c0End); });
         amgInitFinalizeKernel<NCH><<<1, kBlock, 0, s>>>(st);
         enqueuePrecond<P, NCH>(s, rP, z, tol2, 1);
@@ -1652,7 +1677,7 @@ namespace nsfem
         P * z = reinterpret_cast<P *>(z_.get());
         const P * inv = levelMatrix<P>(0).invDiag;
         const int c0End = fusedSweep() ? levels_[0].colorStart[1] : 0;
-        byRowLanes<NCH>(levels_[0].lanes, levels_[0].nnz / n_, [&]<int LN>()
+        byProductLanes<NCH>(levels_[0].lanes, [&]<int LN>()
                         { amgDirectionKernel<P, LN, NCH><<<parts_, kCgBlock<NCH>, 0, s>>>(a64_, z, p_.get(), q_.get(), st); });
         amgUpdateKernel<P, NCH><<<parts_, kCgBlock<NCH>, 0, s>>>(n_, p_.get(), q_.get(), xDevice_, r_.get(), rP, st, z, inv, c0End);
         enqueuePrecond<P, NCH>(s, rP, z, tol2, 0);
@@ -1724,7 +1749,7 @@ namespace nsfem
                       bytes = bDir;
                       launch = [=, this]()
                       {
-                          byRowLanes<NCH>(levels_[0].lanes, levels_[0].nnz / n_, [&]<int LN>()
+                          byProductLanes<NCH>(levels_[0].lanes, [&]<int LN>()
                                   { amgDirectionKernel<P, LN, NCH><<<parts_, kCgBlock<NCH>, 0, s>>>(a64_, z, p_.get(), q_.get(), st); });
                       };
                   }

@@ -208,7 +208,7 @@ namespace
 
 struct nsfem_csr
 {
-    int rows, cols, nnz, dtype, lanes;
+    int rows, cols, nnz, dtype;
     DeviceArray<int> rowStart, column;
     DeviceArray<char> values;
     CsrView view() const { return CsrView{rows, cols, nnz, rowStart.get(), column.get(), values.get(), dtype}; }
@@ -331,7 +331,6 @@ extern "C"
             m->cols = cols;
             m->nnz = nnz;
             m->dtype = dtype;
-            m->lanes = lanesForMeanRow(static_cast<double>(nnz) / rows);
             m->rowStart.upload(h.rowStart);
             m->column.upload(nnz ? h.column : std::vector<int>{0});
             const size_t vb = std::max<size_t>(1, nnz) * dtypeSize(dtype);
@@ -379,7 +378,7 @@ extern "C"
             need(m, "matrix");
             need(x, "x");
             need(y, "y");
-            csrMul(m->view(), numCh, x, ldx, y, ldy, alpha, beta, nullptr, m->rows, lanes > 0 ? lanes : m->lanes, libraryStream());
+            csrMul(m->view(), numCh, x, ldx, y, ldy, alpha, beta, nullptr, m->rows, lanes, libraryStream());
             syncLibraryStream(); });
     }
 

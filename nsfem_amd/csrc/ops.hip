@@ -62,17 +62,63 @@ namespace nsfem
                      const int * rowIds, int outRows, int lanes, hipStream_t s)
         {
             const T * vals = static_cast<const T *>(A.values);
-            auto launch = [&]<int L, int C>(const T * xs, T * ys)
+            auto launch = [&]<int L, int C, int U = 0>(const T * xs, T * ys)
             {
                 const long threads = static_cast<long>(outRows) * L;
                 const int grid = ceilDiv(threads, kBlock);
-                csrMulKernel<T, L, C><<<grid, kBlock, 0, s>>>(outRows, A.rowStart, A.column, vals, xs, ldx, ys, ldy,
+                csrMulKernel<T, L, C, U><<<grid, kBlock, 0, s>>>(outRows, A.rowStart, A.column, vals, xs, ldx, ys, ldy,
                                                               static_cast<T>(alpha), static_cast<T>(beta), rowIds);
             };
+            // lanes = 0: by the mean row length, so that a row is one round of
+            // loads on as few lanes as hold it.  Measured with 250k pressure
+            // nodes, us a call, FP64 / FP32, from lanesForMeanRow's shape:
+            // divergence rows (38 entries) one column 48.8 / 44.4 -> 36.4 /
+            // 31.0, two 55.4 / 50.4 -> 44.2 / 38.3; P2 rows (11.5) one column 64.7 /
+            // 51.9 -> 52.6 / 42.4, two in FP32 60.1 -> 57.0 (in FP64 eight
+            // lanes with one entry stay ahead, 69.6 against 71.1: the gathers of
+            // two columns bound it); P1 rows (7) 17.7 -> 16.6; gradient rows
+            // (4.7) 43.7 -> 41.1.  At 20k nodes all shapes are within 1 us; small
+            // products are one latency long and keep the wider shape, which
+            // reaches more CUs with shorter chains (2,008 divergence rows 13.8 us
+            // a call, 14.0 on eight lanes).
+            const double mean = A.rows > 0 ? static_cast<double>(A.nnz) / A.rows : 1.0;
+            if (lanes == 0 && outRows < 16384)
+            {
+                lanes = lanesForMeanRow(mean);
+            }
             auto byLanes = [&]<int C>(const T * xs, T * ys)
             {
                 switch (lanes)
                 {
+                case 0:
+                    if (mean < 5)
+                    {
+                        launch.template operator()<2, C, 4>(xs, ys);
+                    }
+                    else if (mean < 9)
+                    {
+                        launch.template operator()<4, C, 2>(xs, ys);
+                    }
+                    else if (mean < 16)
+                    {
+                        if constexpr (C == 2 && std::is_same_v<T, double>)
+                        {
+                            launch.template operator()<8, C, 1>(xs, ys);
+                        }
+                        else
+                        {
+                            launch.template operator()<4, C, 8>(xs, ys);
+                        }
+                    }
+                    else if (mean < 48)
+                    {
+                        launch.template operator()<8, C, 4>(xs, ys);
+                    }
+                    else
+                    {
+                        launch.template operator()<64, C>(xs, ys);
+                    }
+                    break;
                 case 4: launch.template operator()<4, C>(xs, ys); break;
                 case 8: launch.template operator()<8, C>(xs, ys); break;
                 case 16: launch.template operator()<16, C>(xs, ys); break;
@@ -110,10 +156,7 @@ namespace nsfem
         {
             return;
         }
-        if (lanes <= 0)
-        {
-            lanes = lanesForMeanRow(A.rows > 0 ? static_cast<double>(A.nnz) / A.rows : 1.0);
-        }
+        lanes = std::max(lanes, 0);
         if (A.dtype == F64)
         {
             csrMulT<double>(A, numCh, x, ldx, y, ldy, alpha, beta, rowIds, outRows, lanes, s);

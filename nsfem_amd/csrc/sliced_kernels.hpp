@@ -355,47 +355,6 @@ namespace nsfem
     constexpr int kWideGroups = 256, kWideGroupsLong = 512;
     constexpr long kWideLong = 8L << 20; // values of a vector from which on two pay
 
-    // The product of the row whose entries are [j0, j1) for the lane's channel,
-    // NCH lanes a row.  The lanes load NCH entries at once and pass them around:
-    // loaded where they are used, values and columns are two of three vector
-    // memory instructions, each as long as a gather, and those bound the kernel
-    // (40k pressure nodes x 16
-    // channels: direction 41 -> 35 us in mixed precision, 51 -> 38 in FP64).
-    // Every lane of the wavefront takes part (the bounds of its loops are
-    // the wavefront's).
-    template <int U, int NCH, typename V, typename X>
-    __device__ __forceinline__ V channelRowDot(int j0, int j1, const int * __restrict__ column, const V * __restrict__ values,
-                                               const X * __restrict__ x)
-    {
-        const int lane = static_cast<int>(threadIdx.x) & 63;
-        const int c = lane % NCH, group = lane - c;
-        constexpr int K = U < NCH ? U : NCH;
-        V acc = V(0);
-        for (int jb = j0; __any(jb < j1); jb += NCH)
-        {
-            const int count = j1 - jb;
-            const int e = c < count ? jb + c : 0; // (entry 0 exists; its term is dropped)
-            const V v = values[e];
-            const int col = column[e];
-            for (int u = 0; u < NCH && __any(u < count); u += K)
-            {
-                X xv[K];
-#pragma unroll
-                for (int k = 0; k < K; k++)
-                {
-                    xv[k] = x[static_cast<long>(__shfl(col, group + u + k, 64)) * NCH + c];
-                }
-#pragma unroll
-                for (int k = 0; k < K; k++)
-                {
-                    const V vk = __shfl(v, group + u + k, 64);
-                    acc = u + k < count ? fmaT(vk, static_cast<V>(xv[k]), acc) : acc;
-                }
-            }
-        }
-        return acc;
-    }
-
     // Rows range.x + t / NCH, + kWideBlock / NCH, ...: own(row) loads the row's
     // operands, part(row, acc) takes its product.  The next row's bounds load
     // with the current row's entries; U entries go out together.  begin() runs
