@@ -794,11 +794,12 @@ namespace nsfem
 
     void ChorinGpu::destroyStepGraph()
     {
-        if (stepExec_)
+        for (StepGraph & g : stepGraphs_)
         {
-            (void)hipGraphExecDestroy(stepExec_);
-            stepExec_ = nullptr;
+            (void)hipGraphExecDestroy(g.exec);
         }
+        stepGraphs_.clear();
+        stepExec_ = nullptr;
     }
 
     void ChorinGpu::setBudgets(int tent, int pres, int fin)
@@ -815,21 +816,43 @@ namespace nsfem
         const int minMargin[3] = {3, amgPressure ? 3 : 16, 3};
         const int slack[3] = {8, amgPressure ? 2 : 8, 8};
         const int frac[3] = {4, 24, 4};
+        auto margin = [&](int k) { return std::max(minMargin[k], counts[k] / frac[k]); };
+        auto fits = [&](int k, int budget)
+        {
+            const int c = counts[k], m = margin(k);
+            return c + m / 2 <= budget && budget <= c + 2 * m + slack[k];
+        };
         bool rebuild = false;
         for (int k = 0; k < 3; k++)
         {
-            const int c = counts[k];
-            const int m = std::max(minMargin[k], c / frac[k]);
-            if (c + m / 2 > budget_[k] || budget_[k] > c + 2 * m + slack[k])
+            rebuild = rebuild || !fits(k, budget_[k]);
+        }
+        if (!rebuild)
+        {
+            return;
+        }
+        // a graph kept from earlier counts, if its budgets fit: a run whose
+        // counts alternate (restarts, a cold first step and warm ones) would
+        // otherwise rebuild its thousands of nodes every few steps (nine meshes
+        // of 5k to 25k nodes restarted every four steps, ~460 pressure
+        // iterations: three to four builds of 15 to 23 ms a pass)
+        for (StepGraph & g : stepGraphs_)
+        {
+            if (fits(0, g.budget[0]) && fits(1, g.budget[1]) && fits(2, g.budget[2]))
             {
-                budget_[k] = c + m;
-                rebuild = true;
+                std::copy(g.budget, g.budget + 3, budget_);
+                stepExec_ = g.exec;
+                return;
             }
         }
-        if (rebuild)
+        for (int k = 0; k < 3; k++)
         {
-            destroyStepGraph();
+            if (!fits(k, budget_[k]))
+            {
+                budget_[k] = counts[k] + margin(k);
+            }
         }
+        stepExec_ = nullptr; // built with the next step
     }
 
     void ChorinGpu::buildStepGraph()
@@ -884,9 +907,18 @@ namespace nsfem
             throw;
         }
         NSFEM_HIP(hipStreamEndCapture(s, &graph));
-        const hipError_t rc = hipGraphInstantiate(&stepExec_, graph, nullptr, nullptr, 0);
+        StepGraph g{};
+        const hipError_t rc = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
         NSFEM_HIP(rc);
+        std::copy(budget_, budget_ + 3, g.budget);
+        if (stepGraphs_.size() >= kStepGraphs)
+        {
+            (void)hipGraphExecDestroy(stepGraphs_.front().exec); // the oldest
+            stepGraphs_.erase(stepGraphs_.begin());
+        }
+        stepGraphs_.push_back(g);
+        stepExec_ = g.exec;
         graphTau_ = tau_;
         graphBuilds_++;
         graphBuildSeconds_ += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
@@ -895,7 +927,7 @@ namespace nsfem
     bool ChorinGpu::stepCaptured(ChorinStepStats * stats)
     {
         const hipStream_t s = libraryStream();
-        if (stepExec_ && graphTau_ != tau_)
+        if (!stepGraphs_.empty() && graphTau_ != tau_)
         {
             destroyStepGraph(); // tau is a parameter of the captured kernels
         }

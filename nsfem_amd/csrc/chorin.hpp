@@ -203,6 +203,15 @@ namespace nsfem
         void setBudgets(int tent, int pres, int fin);
 
         DevCsr nuK_, A_, vpd_, pvd_;
+        // captured steps by their iteration budgets, at most kStepGraphs (the
+        // oldest goes); stepExec_ is the current one, in the list, or null
+        struct StepGraph
+        {
+            hipGraphExec_t exec;
+            int budget[3];
+        };
+        static constexpr size_t kStepGraphs = 4;
+        std::vector<StepGraph> stepGraphs_;
         hipGraphExec_t stepExec_ = nullptr;
         double graphTau_ = -1;
         int budget_[3] = {0, 0, 0}; // tentative, pressure, final iterations
