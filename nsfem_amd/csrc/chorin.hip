@@ -831,14 +831,21 @@ namespace nsfem
         {
             return;
         }
-        // a graph kept from earlier counts, if its budgets fit: a run whose
+        // a graph kept from earlier counts, if its budgets fit with at least
+        // the margin that a new one would get: a run whose
         // counts alternate (restarts, a cold first step and warm ones) would
         // otherwise rebuild its thousands of nodes every few steps (nine meshes
         // of 5k to 25k nodes restarted every four steps, ~460 pressure
         // iterations: three to four builds of 15 to 23 ms a pass)
         for (StepGraph & g : stepGraphs_)
         {
-            if (fits(0, g.budget[0]) && fits(1, g.budget[1]) && fits(2, g.budget[2]))
+            bool good = true;
+            for (int k = 0; k < 3; k++)
+            {
+                const int least = fits(k, budget_[k]) ? 0 : counts[k] + margin(k);
+                good = good && fits(k, g.budget[k]) && g.budget[k] >= least;
+            }
+            if (good)
             {
                 std::copy(g.budget, g.budget + 3, budget_);
                 stepExec_ = g.exec;
