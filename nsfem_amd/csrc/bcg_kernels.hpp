@@ -65,7 +65,11 @@ namespace nsfem
         int rowsPerBlock;   // a multiple of kBlock / NCH
     };
 
-    constexpr int kBcgSmallBlock = 1024;
+    // One thread per entry of the small matrices: 8 columns are one wavefront,
+    // whose barriers cost next to nothing (1,024 threads for any width took 8
+    // and 10.8 us for the step and the direction matrix).
+    template <int NCH>
+    constexpr int kBcgSmallBlock = NCH * NCH < 64 ? 64 : NCH * NCH;
     // The Gram partials of the row blocks are summed in kBcgSlices slices of
     // blocks (b = slice mod kBcgSlices) by as many workgroups per group of 64
     // entries; the small kernels add the slice sums in slice order.
@@ -299,7 +303,7 @@ namespace nsfem
 
     // alpha = (P^T Q)^-1 rho
     template <int NCH>
-    __global__ void __launch_bounds__(kBcgSmallBlock) bcgAlphaKernel(BcgState st)
+    __global__ void __launch_bounds__(kBcgSmallBlock<NCH>) bcgAlphaKernel(BcgState st)
     {
         __shared__ double G[NCH * NCH], B[NCH * NCH], X[NCH * NCH], piv[NCH + 1];
         __shared__ int dropped;
@@ -498,7 +502,7 @@ namespace nsfem
     // stop the iteration: flags[0] = 1, flags[3] = 2 or 1); else beta =
     // rho^-1 rho' and rho = rho'.
     template <int NCH>
-    __global__ void __launch_bounds__(kBcgSmallBlock) bcgBetaKernel(BcgState st, int init)
+    __global__ void __launch_bounds__(kBcgSmallBlock<NCH>) bcgBetaKernel(BcgState st, int init)
     {
         __shared__ double G[NCH * NCH], Rn[NCH * NCH], X[NCH * NCH], piv[NCH + 1];
         __shared__ double worst;
@@ -518,42 +522,36 @@ namespace nsfem
             const int i = e / NCH, k = e % NCH;
             Rn[e] = 0.5 * (X[e] + X[k * NCH + i]); // Z^T R is symmetric up to the preconditioner's rounding
         }
-        if (t == 0)
+        if (t < 64)
         {
-            allDone = 1;
-            bad = 0;
-            worst = 0;
-        }
-        __syncthreads();
-        if (t == 0)
-        {
-            for (int c = 0; c < NCH; c++)
+            // one column per lane of the first wavefront (NCH <= 32)
+            double rr = 0, share = 0;
+            bool open = false, broken = false;
+            if (t < NCH)
             {
-                const double rr = sliceSum(st.normTotal, 2 * NCH, NCH + c);
-                double bb = 0;
+                rr = sliceSum(st.normTotal, 2 * NCH, NCH + t);
+                const double bb = init == 2 ? sliceSum(st.normTotal, 2 * NCH, t) : st.bb[t];
                 if (init == 2)
                 {
-                    bb = sliceSum(st.normTotal, 2 * NCH, c);
+                    st.bb[t] = bb;
                 }
-                if (init == 2)
-                {
-                    st.bb[c] = bb;
-                }
-                else
-                {
-                    bb = st.bb[c];
-                }
-                st.rr[c] = rr;
+                st.rr[t] = rr;
                 const double ref = bb > 0 ? bb : 1.0;
-                if (!(rr <= st.tol2 * ref))
-                {
-                    allDone = 0;
-                }
-                if (!isfinite(rr))
-                {
-                    bad = 1;
-                }
-                worst = fmax(worst, rr / ref);
+                open = !(rr <= st.tol2 * ref);
+                broken = !isfinite(rr);
+                share = rr / ref;
+            }
+            const int anyOpen = __any(open), anyBroken = __any(broken);
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1)
+            {
+                share = fmax(share, __shfl_xor(share, off, 64));
+            }
+            if (t == 0)
+            {
+                allDone = !anyOpen;
+                bad = anyBroken;
+                worst = share;
             }
         }
         __syncthreads();

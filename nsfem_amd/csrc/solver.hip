@@ -577,10 +577,33 @@ namespace nsfem
             throw std::invalid_argument("rowsPerBlock must be >= 0");
         }
         // wide channel tiles run one lane per channel: the lane count is fixed
-        const int L = opt_.numCh > 2 ? opt_.numCh : (lanes > 0 ? lanes : std::min(16, lanesForMeanRow(meanRow_)));
+        // Default lanes of one and two channels: a row in one round of loads while
+        // the launch is a latency long, fewer lanes (every one of them at
+        // work) once there are rows enough.  us per PCG iteration on 8 / 4 / 2
+        // lanes: P2 rows, two channels, 7k rows 59.3 / 61.4 / 66.4, 100k 86.5 /
+        // 79.3 / 81.8, 240k 120 / 109 / 113, 2M 635 / 521 / 523; P1 rows 1.9k 24.7 /
+        // 24.7 / 26.3, 25k 28.5 / 25.1 / 24.7, 60k 32.0 / 28.5 / 26.4.  A batch
+        // keeps the lanes by row length: its rows belong to systems of any size.
+        auto defaultLanes = [&]()
+        {
+            if (flat() && meanRow_ <= 8)
+            {
+                return n_ >= 16384 ? 2 : 4;
+            }
+            return flat() && meanRow_ < 12 && n_ >= 32768 ? 4 : std::min(16, lanesForMeanRow(meanRow_));
+        };
+        const int L = opt_.numCh > 2 ? opt_.numCh : (lanes > 0 ? lanes : defaultLanes());
         const int slab = kBlock / L;
-        // the sweeps write no partial sums: any row count goes
-        int rpb = rowsPerBlock > 0 ? rowsPerBlock : (sweeps ? 4 * slab : std::max(4 * slab, minRowsPerBlock()));
+        // Default rows: a workgroup walks its row slabs one after another, each a
+        // chain of dependent loads, so one slab for one system, whose main map
+        // is widened per kernel kind (setupKindMaps; the sweeps write no partial
+        // sums, so any count goes); a batch's main map is every kernel's, and
+        // its partial sums are re-summed by every workgroup: four.  Measured
+        // against four slabs, us per PCG iteration: 2k pressure nodes velocity
+        // (two columns) 107 -> 59 and pressure 39.9 -> 24.7, 25k 128 -> 87 and
+        // 42.5 -> 28.6, 60k 170 -> 120 and 44.6 -> 32.0, 500k velocity 697 -> 635.
+        const int slabs = flat() ? 1 : 4;
+        int rpb = rowsPerBlock > 0 ? rowsPerBlock : (sweeps ? slabs * slab : std::max(slabs * slab, minRowsPerBlock()));
         rpb = std::max(slab, rpb / slab * slab);
         return {L, rpb};
     }
@@ -653,8 +676,9 @@ namespace nsfem
         rowsDir_ = rowsUpd_ = rowsRho_ = 0;
         lanesDir_ = 0;
         setupKindMaps();
-        // the sweeps take the same shape until reshapeSweeps
-        reshapeSweeps(lanes_, rowsPerBlock_);
+        // the sweeps take the same shape until reshapeSweeps (one system's:
+        // their own default rows with a default shape)
+        reshapeSweeps(lanes_, rowsPerBlock > 0 || !flat() ? rowsPerBlock_ : 0);
     }
 
     void McgsSolver::setupMainMap()
@@ -2043,7 +2067,7 @@ namespace nsfem
                          constexpr int red = (C * C + 63) / 64 + 1;
                          bcgProductKernel<double, C><<<g, kBlock, 0, s>>>(A, b, p64_.get(), q64_.get());
                          bcgGramReduceKernel<C><<<(red - 1) * kBcgSlices, kBlock, 0, s>>>(b, 0);
-                         bcgAlphaKernel<C><<<1, kBcgSmallBlock, 0, s>>>(b);
+                         bcgAlphaKernel<C><<<1, kBcgSmallBlock<C>, 0, s>>>(b);
                          bcgUpdateKernel<double, P, C><<<g, kBlock, 0, s>>>(b, M.invDiag, p64_.get(), q64_.get(), x64_.get(), r64_.get(),
                                                                              rP, z, color0End_);
                      });
@@ -2053,7 +2077,7 @@ namespace nsfem
                          constexpr int red = (C * C + 63) / 64 + 1;
                          bcgRhoKernel<P, double, C><<<g, kBlock, 0, s>>>(M, b, rP, r64_.get(), z, color0End_);
                          bcgGramReduceKernel<C><<<red * kBcgSlices, kBlock, 0, s>>>(b, 1);
-                         bcgBetaKernel<C><<<1, kBcgSmallBlock, 0, s>>>(b, 0);
+                         bcgBetaKernel<C><<<1, kBcgSmallBlock<C>, 0, s>>>(b, 0);
                          bcgDirectionKernel<double, P, C><<<g, kBlock, 0, s>>>(b, z, p64_.get(), 0);
                      });
     }
@@ -2101,7 +2125,7 @@ namespace nsfem
                              constexpr int red = (C * C + 63) / 64 + 1;
                              bcgRhoKernel<P, double, C><<<g, kBlock, 0, s>>>(M, b, rP, r64_.get(), z, color0End_);
                              bcgGramReduceKernel<C><<<red * kBcgSlices, kBlock, 0, s>>>(b, 1);
-                             bcgBetaKernel<C><<<1, kBcgSmallBlock, 0, s>>>(b, first ? 2 : 1);
+                             bcgBetaKernel<C><<<1, kBcgSmallBlock<C>, 0, s>>>(b, first ? 2 : 1);
                              bcgDirectionKernel<double, P, C><<<g, kBlock, 0, s>>>(b, z, p64_.get(), 1);
                          });
             NSFEM_HIP(hipGetLastError());
