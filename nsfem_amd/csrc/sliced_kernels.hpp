@@ -13,7 +13,7 @@
 //
 // Bound by the matrix stream; on the P2 mass matrix with 2M rows, FP64 with the
 // FP32 factor, two channels: direction 95 us (420 MB algorithmic, 4.4 TB/s;
-// 476 MB of traffic), each of the factor's launches 41 us (156 MB, 3.8 TB/s),
+// 486 MB of traffic), each of the factor's launches 41 us (156 MB, 3.8 TB/s),
 // an iteration 224 us.  The lane-split kernels on colour-major rows took 160,
 // 56 and 341 us at their best launch shape, 220, 141 and 585 us at the
 // default one: a row's gathers came from up to seven colour regions, and the
