@@ -1,0 +1,49 @@
+"""Default launch shapes of one system's solvers (lanes by rows and row length,
+one row slab per workgroup) against an explicit shape, at the lines of the rule."""
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+pytestmark = pytest.mark.gpu
+
+
+def _band(n, half):
+    """Symmetric band with 2 half off-diagonals, diagonally dominant: condition
+    below 5 after scaling by the diagonal."""
+    rng = np.random.default_rng(n + half)
+    d = {}
+    for k in range(1, min(half, n - 1) + 1):
+        d[k] = d[-k] = -rng.uniform(0.5, 1, n - k)
+    a = sp.diags(list(d.values()), list(d.keys()), shape=(n, n)).tocsr() if d else sp.csr_matrix((n, n))
+    return (a + sp.diags(1.5 * np.asarray(abs(a).sum(axis=1)).ravel() + 1)).tocsr()
+
+
+# half 3: 6 off-diagonal entries, 4 lanes below 16,384 rows and 2 from there;
+# 5: 10 entries, 8 lanes below 32,768 rows and 4 from there; 9: 18 entries, 16 lanes
+@pytest.mark.parametrize("n,half", [(1, 0), (33, 3), (255, 5), (257, 9), (16383, 3), (16384, 3), (32767, 5), (32768, 5), (40001, 9)])
+@pytest.mark.parametrize("name,nch,dtype", [("pcg", 1, np.float64), ("pcg", 2, np.float64), ("pcg_mixed", 2, np.float64),
+                                            ("gs", 2, np.float32), ("pcg", 8, np.float64)])
+def test_default_shape_equals_an_explicit_one(n, half, name, nch, dtype):
+    from nsfem_amd import cu
+    a = _band(n, half)
+    b = np.random.default_rng(3).uniform(-1, 1, nch * n).astype(dtype)
+    target = 1e-12 if dtype == np.float64 else 1e-4
+    xs = []
+    for shape in (None, (8, 128)):
+        s = cu.createSolver(name, nch, a, 300, target, 1, dtype=dtype)
+        if shape:
+            s.reshape(*shape)
+        s.getRhs().upload(b)
+        s.getSol().memsetZero()
+        s.solve()
+        xs.append(s.getSol().download().astype(np.float64))
+    # true residuals: the pcg target is relative to |b|, gs' the root mean
+    # square over a column (summed over the columns at most); rounding of the
+    # result adds a few ulps of |A||x|
+    for x in xs:
+        for c in range(nch):
+            bc, xc = b[c * n:(c + 1) * n].astype(np.float64), x[c * n:(c + 1) * n]
+            bound = 1.01 * target * (np.sqrt(n * nch) if name == "gs" else np.linalg.norm(bc))
+            bound += 8 * np.finfo(dtype).eps * np.linalg.norm(abs(a) @ abs(xc))
+            assert np.linalg.norm(bc - a @ xc) <= bound
