@@ -1394,9 +1394,11 @@ extern "C"
             need(ch, "chorin");
             need(key, "key");
             if (which < 0 || which > 2) throw std::invalid_argument("which must be 0 (velocity), 1 (pressure) or 2 (both)");
+            // before the change: it frees buffers that captured steps hold, also
+            // where the second solver then rejects it
+            ch->core->invalidateStepGraph();
             if (which != 1) applySolverOption(ch->core->velocitySolver(), key, value);
-            if (which != 0) applySolverOption(ch->core->pressureSolver(), key, value);
-            ch->core->invalidateStepGraph(); });
+            if (which != 0) applySolverOption(ch->core->pressureSolver(), key, value); });
     }
 
     int nsfem_chorin_autotune(nsfem_chorin * ch, int reps, int * shape)
@@ -1405,6 +1407,8 @@ extern "C"
                        {
             need(ch, "chorin");
             if (reps < 1) throw std::invalid_argument("reps must be positive");
+            // new launch shapes free the partial sums that captured steps hold
+            ch->core->invalidateStepGraph();
             // block PCG keeps its fixed shapes
             for (McgsSolver * sv : {&ch->core->velocitySolver(), &ch->core->pressureSolver()})
             {
