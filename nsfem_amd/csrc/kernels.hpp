@@ -129,7 +129,7 @@ namespace nsfem
     // Plain CSR products: y = alpha * A x (+ beta y), NCH planar channels.
     // rowIds != nullptr: output row i is A's row rowIds[i] (fused gather).
     // ------------------------------------------------------------------
-    // U: entries per lane and step (0: from the lanes, as below).
+    // UNROLL: entries per lane and step (0: from the lanes, as below).
     template <typename T, int LANES, int NCH, int UNROLL = 0>
     __global__ void __launch_bounds__(kBlock) csrMulKernel(int rows, const int * __restrict__ rowStart,
                                                             const int * __restrict__ column, const T * __restrict__ values,

@@ -69,62 +69,90 @@ namespace nsfem
                 csrMulKernel<T, L, C, U><<<grid, kBlock, 0, s>>>(outRows, A.rowStart, A.column, vals, xs, ldx, ys, ldy,
                                                               static_cast<T>(alpha), static_cast<T>(beta), rowIds);
             };
-            // lanes = 0: by the mean row length, so that a row is one round of
-            // loads on as few lanes as hold it.  Measured with 250k pressure
-            // nodes, us a call, FP64 / FP32, from lanesForMeanRow's shape:
-            // divergence rows (38 entries) one column 48.8 / 44.4 -> 36.4 /
-            // 31.0, two 55.4 / 50.4 -> 44.2 / 38.3; P2 rows (11.5) one column 64.7 /
-            // 51.9 -> 52.6 / 42.4, two in FP32 60.1 -> 57.0 (in FP64 eight
-            // lanes with one entry stay ahead, 69.6 against 71.1: the gathers of
-            // two columns bound it); P1 rows (7) 17.7 -> 16.6; gradient rows
-            // (4.7) 43.7 -> 41.1.  At 20k nodes all shapes are within 1 us; small
-            // products are one latency long and keep the wider shape, which
-            // reaches more CUs with shorter chains (2,008 divergence rows 13.8 us
-            // a call, 14.0 on eight lanes).
-            const double mean = A.rows > 0 ? static_cast<double>(A.nnz) / A.rows : 1.0;
-            if (lanes == 0 && outRows < 16384)
+            auto byLanes = [&]<int C>(int count, const T * xs, T * ys)
             {
-                lanes = lanesForMeanRow(mean);
-            }
-            auto byLanes = [&]<int C>(const T * xs, T * ys)
-            {
-                switch (lanes)
+                switch (count)
                 {
-                case 0:
-                    if (mean < 5)
-                    {
-                        launch.template operator()<2, C, 4>(xs, ys);
-                    }
-                    else if (mean < 9)
-                    {
-                        launch.template operator()<4, C, 2>(xs, ys);
-                    }
-                    else if (mean < 16)
-                    {
-                        if constexpr (C == 2 && std::is_same_v<T, double>)
-                        {
-                            launch.template operator()<8, C, 1>(xs, ys);
-                        }
-                        else
-                        {
-                            launch.template operator()<4, C, 8>(xs, ys);
-                        }
-                    }
-                    else if (mean < 48)
-                    {
-                        launch.template operator()<8, C, 4>(xs, ys);
-                    }
-                    else
-                    {
-                        launch.template operator()<64, C>(xs, ys);
-                    }
-                    break;
                 case 4: launch.template operator()<4, C>(xs, ys); break;
                 case 8: launch.template operator()<8, C>(xs, ys); break;
                 case 16: launch.template operator()<16, C>(xs, ys); break;
                 case 32: launch.template operator()<32, C>(xs, ys); break;
                 case 64: launch.template operator()<64, C>(xs, ys); break;
                 default: throw std::invalid_argument("lanes must be 4, 8, 16, 32 or 64");
+                }
+            };
+            // lanes = 0: lanesForMeanRow's shape, which suits a launch that is one
+            // latency long (short chains, many CUs), until the rows are so many
+            // that idle lanes count; then fewer lanes with more loads in flight.
+            // A row count where a shape is ahead on every measured matrix of
+            // its bin is the line: P1, P2, divergence and gradient matrices of
+            // 4.5k to 250k pressure nodes (and matrices of scattered columns,
+            // "scattered").  us a call, from lanesForMeanRow's shape:
+            // - gradient rows (4.7): two lanes of four entries, FP64 only, 483k
+            //   rows one column 21.6 -> 20.8, two 23.1 -> 22.6; 2M 43.4 -> 40.6
+            //   and 50.5 -> 48.9; in FP32 and below they lose 2 to 9 %;
+            // - P1 rows (7): four lanes, 35k 14.1 -> 14.0, 251k one column FP64
+            //   17.7 -> 16.6, two 19.9 -> 18.4 (below 32k the same);
+            // - P2 rows (9 and 19 entries, 11.3 to 11.5 in the mean): three
+            //   entries a lane, which hold a short row at once, on eight lanes
+            //   in FP64 (80k rows 16.5 -> 16.4, 1M 65.4 -> 51.0) and four in
+            //   FP32 (80k 15.7 -> 14.9, 1M 52.7 -> 41.7, two columns 60.9 ->
+            //   51.5); two columns in FP64 keep eight lanes of one;
+            //   scattered rows of 11 entries lose 2 to 13 % on them;
+            // - 12 to 24 (scattered only): eight lanes of one entry, 13 entries
+            //   160k rows 1.07 to 1.10 times as fast, 20 entries 0.98 to 1.05;
+            // - divergence rows (38): sixteen lanes below 65k rows, 20k 15.9
+            //   -> 15.1, 35k 17.5 -> 16.5, above eight lanes of four entries,
+            //   121k 31.6 -> 25.8, 251k 49.5 -> 36.7, two columns 54.9 -> 44.3.
+            const double mean = A.rows > 0 ? static_cast<double>(A.nnz) / A.rows : 1.0;
+            auto byRows = [&]<int C>(const T * xs, T * ys)
+            {
+                constexpr bool f64 = std::is_same_v<T, double>;
+                if constexpr (f64)
+                {
+                    if (mean >= 4 && mean < 5 && outRows >= 393216)
+                    {
+                        launch.template operator()<2, C, 4>(xs, ys);
+                        return;
+                    }
+                }
+                if constexpr (!f64 || C == 1)
+                {
+                    if (mean >= 11 && mean < 12 && outRows >= 65536)
+                    {
+                        launch.template operator()<f64 ? 8 : 4, C, 3>(xs, ys);
+                        return;
+                    }
+                }
+                if (mean >= 24 && mean < 48 && outRows >= 65536)
+                {
+                    launch.template operator()<8, C, 4>(xs, ys);
+                    return;
+                }
+                int count = lanesForMeanRow(mean);
+                if (mean >= 5 && mean < 9 && outRows >= 32768)
+                {
+                    count = 4;
+                }
+                else if (mean >= 12 && mean < 24 && outRows >= 65536)
+                {
+                    count = 8;
+                }
+                else if (mean >= 24 && mean < 48 && outRows >= 16384)
+                {
+                    count = 16;
+                }
+                byLanes.template operator()<C>(count, xs, ys);
+            };
+            auto run = [&]<int C>(const T * xs, T * ys)
+            {
+                if (lanes == 0)
+                {
+                    byRows.template operator()<C>(xs, ys);
+                }
+                else
+                {
+                    byLanes.template operator()<C>(lanes, xs, ys);
                 }
             };
             // Channels are processed two at a time (the matrix is read once per pair).
@@ -134,11 +162,11 @@ namespace nsfem
                 T * ys = static_cast<T *>(y) + static_cast<long>(c0) * ldy;
                 if (numCh - c0 >= 2)
                 {
-                    byLanes.template operator()<2>(xs, ys);
+                    run.template operator()<2>(xs, ys);
                 }
                 else
                 {
-                    byLanes.template operator()<1>(xs, ys);
+                    run.template operator()<1>(xs, ys);
                 }
             }
             NSFEM_HIP(hipGetLastError());
