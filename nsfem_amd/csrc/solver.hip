@@ -602,7 +602,27 @@ namespace nsfem
         // against four slabs, us per PCG iteration: 2k pressure nodes velocity
         // (two columns) 107 -> 59 and pressure 39.9 -> 24.7, 25k 128 -> 87 and
         // 42.5 -> 28.6, 60k 170 -> 120 and 44.6 -> 32.0, 500k velocity 697 -> 635.
-        const int slabs = flat() ? 1 : 4;
+        // From eight columns on the sums that every workgroup of the next kernel
+        // (or the finalize) adds up, columns x workgroups, come to outweigh the
+        // chains, and one slab gives way to two and four (the sweeps keep one).
+        // One / two / four slabs: P1 60k rows x 8 57.7 / 54.8 / 56.0, 20k x 16 51.9 /
+        // 49.9 / 50.0, 60k x 16 99.5 / 87.2 / 82.0, 6k x 32 66.7 / 46.8 / 45.7, 60k x
+        // 32 179 / 179 / 149 (with finalize launches 325 / 229 / 204); P2 240k x 16
+        // the same (444 / 370 / 339); few sums, P1 6k x 8 29.3 / 32.5 / 39.7.
+        auto defaultSlabs = [&]()
+        {
+            if (!flat())
+            {
+                return 4;
+            }
+            const long sums = static_cast<long>(ceilDiv(n_, slab)) * opt_.numCh;
+            if (sweeps || opt_.numCh <= 4 || sums <= 12288)
+            {
+                return 1;
+            }
+            return opt_.numCh == 8 || sums <= 32768 ? 2 : 4;
+        };
+        const int slabs = defaultSlabs();
         int rpb = rowsPerBlock > 0 ? rowsPerBlock : (sweeps ? slabs * slab : std::max(slabs * slab, minRowsPerBlock()));
         rpb = std::max(slab, rpb / slab * slab);
         return {L, rpb};

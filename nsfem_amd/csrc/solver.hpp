@@ -255,7 +255,7 @@ namespace nsfem
 
         // Launch shape: lanes per matrix row (1, 2, 4, 8, 16; 0 picks from the mean
         // row length; wide channel tiles always run one lane per channel) and
-        // rows per workgroup (0: four row slabs, for wide tiles at least
+        // rows per workgroup (0: resolveShape's default, for wide tiles at least
         // minRowsPerBlock()).  Rebuilds the block map only; the colouring and
         // matrices are kept.
         void reshape(int lanes, int rowsPerBlock);

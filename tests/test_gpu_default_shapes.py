@@ -47,3 +47,26 @@ def test_default_shape_equals_an_explicit_one(n, half, name, nch, dtype):
             bound = 1.01 * target * (np.sqrt(n * nch) if name == "gs" else np.linalg.norm(bc))
             bound += 8 * np.finfo(dtype).eps * np.linalg.norm(abs(a) @ abs(xc))
             assert np.linalg.norm(bc - a @ xc) <= bound
+
+
+# columns x workgroups of one slab (256 / columns rows) on both sides of 12,288
+# and, from 16 columns on, 32,768: one, two and four slabs
+@pytest.mark.parametrize("n,nch,slabs", [(49152, 8, 1), (49153, 8, 2), (12288, 16, 1), (12289, 16, 2), (32768, 16, 2), (32769, 16, 4),
+                                         (3072, 32, 1), (3073, 32, 2), (8192, 32, 2), (8193, 32, 4), (200001, 4, 1)])
+@pytest.mark.parametrize("name", ["pcg_mixed", "gs"])
+def test_default_slabs_of_wide_tiles(n, nch, slabs, name):
+    from nsfem_amd import cu
+    a = _band(n, 3)
+    b = np.random.default_rng(4).uniform(-1, 1, (nch, n))
+    target = 1e-11
+    s = cu.createSolver(name, nch, a, 300, target, 1)
+    assert s.shape() == (nch, slabs * 256 // nch) and s.sweepShape() == (nch, 256 // nch)
+    s.getRhs().upload(b.ravel())
+    s.getSol().memsetZero()
+    s.solve()
+    x = s.getSol().download().reshape(nch, n)
+    # true residuals, bounded as above
+    for c in range(nch):
+        bound = 1.01 * target * (np.sqrt(n * nch) if name == "gs" else np.linalg.norm(b[c]))
+        bound += 8 * np.finfo(np.float64).eps * np.linalg.norm(abs(a) @ abs(x[c]))
+        assert np.linalg.norm(b[c] - a @ x[c]) <= bound
