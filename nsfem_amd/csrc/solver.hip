@@ -663,12 +663,17 @@ namespace nsfem
         std::vector<int> blockSystem;
         buildBlocks(chunks_, rpb, blocks, blockSystem, colorSweepBlockStart_);
         sweepBlocks_.upload(blocks.empty() ? std::vector<int4>{int4{0, 0, 0, 0}} : blocks);
-        sweepBm_ = bm_;
-        sweepBm_.blocks = sweepBlocks_.get();
-        sweepBm_.numBlocks = static_cast<int>(blocks.size());
-        sweepBm_.rowsPerBlock = rpb;
         destroyGraphs();
         syncLibraryStream();
+    }
+
+    BlockMap McgsSolver::sweepMap() const
+    {
+        BlockMap m = bm_;
+        m.blocks = sweepBlocks_.get();
+        m.numBlocks = colorSweepBlockStart_.back();
+        m.rowsPerBlock = sweepRows_;
+        return m;
     }
 
     void McgsSolver::destroyGraphs()
@@ -1561,7 +1566,7 @@ namespace nsfem
                 }
                 dispatchLC(sweepLanes_, nch, [&]<int L, int C>()
                            {
-                               mcgsColorKernel<T, L, C><<<cnt, kBlock, 0, s>>>(Av, sweepBm_, colorSweepBlockStart_[c], colorRowStart_[c],
+                               mcgsColorKernel<T, L, C><<<cnt, kBlock, 0, s>>>(Av, sweepMap(), colorSweepBlockStart_[c], colorRowStart_[c],
                                                                               colorRowStart_[c + 1], st, b, x, 0);
                            });
             }
@@ -1650,7 +1655,7 @@ namespace nsfem
             }
             dispatchLC(sweepLanes_, nch, [&]<int L, int C>()
                        {
-                           mcgsColorKernel<P, L, C><<<cnt, kBlock, 0, s>>>(M, sweepBm_, colorSweepBlockStart_[c], colorRowStart_[c],
+                           mcgsColorKernel<P, L, C><<<cnt, kBlock, 0, s>>>(M, sweepMap(), colorSweepBlockStart_[c], colorRowStart_[c],
                                                                           colorRowStart_[c + 1], st, r, z, 1);
                        });
         }
@@ -1664,7 +1669,7 @@ namespace nsfem
             }
             dispatchLC(sweepLanes_, nch, [&]<int L, int C>()
                        {
-                           mcgsColorKernel<P, L, C><<<cnt, kBlock, 0, s>>>(M, sweepBm_, colorSweepBlockStart_[c], colorRowStart_[c],
+                           mcgsColorKernel<P, L, C><<<cnt, kBlock, 0, s>>>(M, sweepMap(), colorSweepBlockStart_[c], colorRowStart_[c],
                                                                           colorRowStart_[c + 1], st, r, z, 0);
                        });
         }

@@ -405,7 +405,8 @@ namespace nsfem
         int sweepLanes_ = 8, sweepRows_ = 0;
         std::vector<int> colorSweepBlockStart_;
         DeviceArray<int4> sweepBlocks_;
-        BlockMap sweepBm_{};
+        // (made for each launch from bm_, whose tables other calls reallocate)
+        BlockMap sweepMap() const;
         std::pair<int, int> resolveShape(int lanes, int rowsPerBlock, bool sweeps) const;
         void buildBlocks(const std::vector<RowChunk> & chunks, int rpb, std::vector<int4> & blocks, std::vector<int> & blockSystem,
                          std::vector<int> & colorStart) const;

@@ -105,3 +105,24 @@ def test_preconditioner_switched_off_again_and_refinement_keep_working():
         s.solve()
         x = s.getSol().download()
         assert np.linalg.norm(x - ref) <= 20 * 1e-11 * np.linalg.norm(ref), (precond, restart)
+
+
+@pytest.mark.parametrize("sizes", [[3000], [700, 64, 1300]])
+@pytest.mark.parametrize("name,nch", [("pcg", 2), ("pcg_mixed", 4)])
+def test_sweeps_after_a_change_of_preconditioner_equal_a_fresh_solver(sizes, name, nch):
+    """The colour sweeps' own shape, kept while the approximate inverse and back
+    reallocates the block tables."""
+    from nsfem_amd import cu
+    mats = [_spd(n, 50 + n, "sparse") for n in sizes]
+    b = np.random.default_rng(11).uniform(-1, 1, nch * sum(sizes))
+    xs = []
+    for switched in (False, True):
+        s = cu.createSolver(name, nch, mats[0], 400, 1e-11, 1) if len(mats) == 1 else cu.createBatchSolver(name, nch, mats, 400, 1e-11, 1)
+        s.reshapeSweeps(nch if nch > 2 else 4, 256)
+        for kind in (1, 0) if switched else ():
+            s.setOption("preconditioner", kind)
+        s.getRhs().upload(b)
+        s.getSol().memsetZero()
+        s.solve()
+        xs.append(s.getSol().download())
+    assert np.array_equal(*xs)
