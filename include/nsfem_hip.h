@@ -220,16 +220,13 @@ int nsfem_solver_set_mse_check_interval(nsfem_solver * s, int interval);
  *                  chosen: two parallel launches per application instead of
  *                  2 colours - 2 dependent sweeps (the P2 mass matrix: 12
  *                  iterations where GS takes 13).  Its solves run on a copy
- *                  of the system in locality order; with fused reductions and
- *                  1 or 2 channels on slices of 64 rows with a launch shape
- *                  of their own, so the row counts and lanes of the options
- *                  above (and autotune's) do not reach their kernels.
- *   "rowsPreconditioner" fused reductions on one system, preconditioner
- *                  1: rows per workgroup of the approximate inverse's two
- *                  launches on a region-major map of their own (a positive
- *                  multiple of 256); 0 (default) shares the direction
- *                  kernel's map.  Accepted without effect on 1 and 2
- *                  channels, whose launches run on slices of 64 rows.
+ *                  of the system in locality order, with fused reductions on
+ *                  a launch shape of their own (1 or 2 channels: slices of 64
+ *                  rows), so the row counts and lanes of the options above do
+ *                  not reach their kernels.
+ *   "rowsPreconditioner" 0 or a positive multiple of 256, without effect
+ *                  (the approximate inverse's launches share the direction
+ *                  kernel's workgroups).
  *   "amgChebyshevFrom", "amgChebyshevDegree", "amgChebyshevFraction"
  *                  amg_pcg: the V-cycle levels from this one on (but the
  *                  dense coarsest) are smoothed by this many steps of the
@@ -276,7 +273,8 @@ int nsfem_solver_shape(const nsfem_solver * s, int * lanes, int * rowsPerBlock);
 int nsfem_solver_reshape_sweeps(nsfem_solver * s, int lanes, int rowsPerBlock);
 int nsfem_solver_sweep_shape(const nsfem_solver * s, int * lanes, int * rowsPerBlock);
 /* Rows per workgroup of the direction, update and rho kernels (the main
- * shape's unless fused reductions give them their own). */
+ * shape's unless fused reductions give them their own; direction and update 0
+ * where the approximate inverse's solves run on workgroups of their own). */
 int nsfem_solver_kind_rows(const nsfem_solver * s, int * direction, int * update, int * rho);
 int nsfem_solver_autotune(nsfem_solver * s, int reps, int * lanes, int * rowsPerBlock);
 int nsfem_solver_coloring(const nsfem_solver * s, int system, int * coloring, int * partitionStart);

@@ -148,8 +148,8 @@ namespace
         {
             if (!(value >= 0 && value <= 1 << 20)) throw std::invalid_argument(k + " must be in [0, 2^20]");
             const int v = static_cast<int>(value);
-            solver.setKindRows(k == "rowsDirection" ? v : solver.kindRows(0), k == "rowsUpdate" ? v : solver.kindRows(1),
-                               k == "rowsRho" ? v : solver.kindRows(2));
+            solver.setKindRows(k == "rowsDirection" ? v : solver.laneSplitRows(0), k == "rowsUpdate" ? v : solver.laneSplitRows(1),
+                               k == "rowsRho" ? v : solver.laneSplitRows(2));
         }
         else
         {

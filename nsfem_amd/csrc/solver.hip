@@ -803,10 +803,6 @@ namespace nsfem
         {
             throw std::invalid_argument("rowsPreconditioner must be 0 or a positive multiple of 256");
         }
-        NSFEM_HIP(hipStreamSynchronize(stream_));
-        rowsPrecond_ = rows;
-        setupKindMaps();
-        destroyGraphs();
     }
 
     void McgsSolver::setDirectionLanes(int lanes)
@@ -832,7 +828,9 @@ namespace nsfem
         destroyGraphs();
     }
 
-    int McgsSolver::kindRows(int kind) const
+    int McgsSolver::kindRows(int kind) const { return ownMap() && kind != 2 ? 0 : laneSplitRows(kind); }
+
+    int McgsSolver::laneSplitRows(int kind) const
     {
         if (!(fused() && flat()))
         {
@@ -901,33 +899,19 @@ namespace nsfem
             bmDir_ = flatMap(rowsDir_, nbDir_, 1024);
             bmUpd_ = flatMap(rowsUpd_, nbUpd_, 1024);
             bmRho_ = flatMap(rowsRho_, nbRho_, 4096);
-            const bool ownPrecondMap = rowsPrecond_ > 0 && rowsPrecond_ != bmDir_.rowsPerBlock;
-            if (ownPrecondMap)
-            {
-                bmPre_ = flatMap(rowsPrecond_, nbPre_, 1024);
-            }
             if (regionDir_ && n_ > 0 && !local())
             {
                 regionMap(bmDir_, nbDir_, dirTable_);
-                if (ownPrecondMap)
-                {
-                    regionMap(bmPre_, nbPre_, preTable_);
-                }
-            }
-            if (!ownPrecondMap)
-            {
-                bmPre_ = bmDir_;
-                nbPre_ = nbDir_;
             }
             color0BlocksRho_ = (color0End_ + bmRho_.rowsPerBlock - 1) / bmRho_.rowsPerBlock;
         }
         else
         {
-            bmDir_ = bmUpd_ = bmRho_ = bmPre_ = bm_;
-            nbDir_ = nbUpd_ = nbRho_ = nbPre_ = numBlocks_;
+            bmDir_ = bmUpd_ = bmRho_ = bm_;
+            nbDir_ = nbUpd_ = nbRho_ = numBlocks_;
             color0BlocksRho_ = color0Blocks_;
         }
-        if (sliced() || wideLocal())
+        if (ownMap())
         {
             setupSliceMaps();
             maxBlocks = std::max(maxBlocks, nbDir_);
@@ -1163,14 +1147,14 @@ namespace nsfem
         loc_.rows = BlockMap{loc_.rowBlocks.get(), loc_.sysBlockStart.get(), nullptr, systemRows_.get(), numSystems_, nb, 0, 0, nullptr};
         loc_.slices = loc_.rows;
         loc_.slices.blocks = loc_.sliceBlocks.get();
-        // the reported rows per workgroup stay those of the lane-split maps
-        for (BlockMap * m : {&bmDir_, &bmUpd_, &bmPre_})
+        // (with the lane-split maps' rows per workgroup: laneSplitRows)
+        for (BlockMap * m : {&bmDir_, &bmUpd_})
         {
-            const int reported = m->rowsPerBlock;
+            const int rowsPerBlock = m->rowsPerBlock;
             *m = loc_.rows;
-            m->rowsPerBlock = reported;
+            m->rowsPerBlock = rowsPerBlock;
         }
-        nbDir_ = nbUpd_ = nbPre_ = nb;
+        nbDir_ = nbUpd_ = nb;
     }
 
     template <typename F>
@@ -1283,8 +1267,8 @@ namespace nsfem
                       {
                           auto go = [&]<int C>()
                           {
-                              slicedLowerKernel<P, W, C><<<nbPre_, 64 * W, 0, s>>>(loc_.lower.view<P>(), v.G.diag, loc_.slices, st, v.rP, v.t);
-                              slicedUpperKernel<P, T, W, C><<<nbPre_, 64 * W, 0, s>>>(loc_.upper.view<P>(), v.G.diag, loc_.slices, st, v.t,
+                              slicedLowerKernel<P, W, C><<<nbDir_, 64 * W, 0, s>>>(loc_.lower.view<P>(), v.G.diag, loc_.slices, st, v.rP, v.t);
+                              slicedUpperKernel<P, T, W, C><<<nbDir_, 64 * W, 0, s>>>(loc_.upper.view<P>(), v.G.diag, loc_.slices, st, v.t,
                                                                                      v.z, v.r);
                           };
                           nch == 1 ? go.template operator()<1>() : go.template operator()<2>();
@@ -1297,16 +1281,16 @@ namespace nsfem
                       {
                           if constexpr (kWide<C>)
                           {
-                              wideLowerKernel<P, C><<<nbPre_, kWideBlock, 0, s>>>(v.G, loc_.rows, st, v.rP, v.t);
-                              wideUpperKernel<P, T, C><<<nbPre_, kWideBlock, 0, s>>>(v.G, loc_.rows, st, v.t, v.z, v.r);
+                              wideLowerKernel<P, C><<<nbDir_, kWideBlock, 0, s>>>(v.G, loc_.rows, st, v.rP, v.t);
+                              wideUpperKernel<P, T, C><<<nbDir_, kWideBlock, 0, s>>>(v.G, loc_.rows, st, v.t, v.z, v.r);
                           }
                       });
             return;
         }
         dispatchLC(directionLanes(), nch, [&]<int L, int C>()
                    {
-                       fsaiLowerKernel<P, L, C><<<nbPre_, kBlock, 0, s>>>(v.G, bmPre_, st, v.rP, v.t);
-                       fsaiUpperKernel<P, T, L, C><<<nbPre_, kBlock, 0, s>>>(v.G, bmPre_, st, v.t, v.z, v.r);
+                       fsaiLowerKernel<P, L, C><<<nbDir_, kBlock, 0, s>>>(v.G, bmDir_, st, v.rP, v.t);
+                       fsaiUpperKernel<P, T, L, C><<<nbDir_, kBlock, 0, s>>>(v.G, bmDir_, st, v.t, v.z, v.r);
                    });
     }
 

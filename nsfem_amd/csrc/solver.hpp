@@ -201,13 +201,14 @@ namespace nsfem
         // partials are redone by every block of the next kernel, so fewer,
         // larger blocks pay there.  reshape resets them.
         void setKindRows(int direction, int update, int rho);
-        // Rows per workgroup of the approximate inverse's two launches
-        // (preconditioner = 1; fused reductions on one system, wide tiles): 0
-        // (default) shares the direction kernel's map, else a positive multiple
-        // of 256; no effect on sliced rows (1 and 2 channels).
+        // Accepts 0 and positive multiples of 256 and has no effect: the
+        // approximate inverse's launches share the direction kernel's map.
         void setPreconditionerRows(int rows);
-        int preconditionerRows() const { return rowsPrecond_; }
-        int kindRows(int kind) const; // 0 direction, 1 update, 2 rho
+        // kind: 0 direction, 1 update, 2 rho.  What the kernels run on, 0 where
+        // that is the approximate inverse's own map (ownMap()) ...
+        int kindRows(int kind) const;
+        // ... and what the lane-split kernels take whenever they run
+        int laneSplitRows(int kind) const;
         // Lanes per row of the direction kernel alone (0: the main shape's;
         // 1 and 2 channels).  reshape resets it.
         void setDirectionLanes(int lanes);
@@ -316,7 +317,7 @@ namespace nsfem
         int zColour0End() const { return precond_ == 0 ? color0End_ : 0; }
         // blocks whose rho partials the next direction kernel sums (the
         // approximate inverse runs on the direction kernel's map)
-        int rhoParts() const { return precond_ == 0 ? nbRho_ : nbPre_; }
+        int rhoParts() const { return precond_ == 0 ? nbRho_ : nbDir_; }
         template <typename P>
         McgsMatrix<P> fsaiView() const;
         // The approximate inverse needs no colour order: its solves run on a
@@ -327,6 +328,8 @@ namespace nsfem
         bool sliced() const { return local() && fused() && opt_.numCh <= 2; }
         // ... and on more channels in workgroups of 1,024 threads (wideRows)
         bool wideLocal() const { return local() && fused() && opt_.numCh > 2; }
+        // ... both on a map that the launch-shape options do not reach
+        bool ownMap() const { return sliced() || wideLocal(); }
         void buildLocal(const std::vector<int> & rowStart, const std::vector<int> & rowSplit, const std::vector<int> & column,
                         const std::vector<double> & values, const std::vector<double> & diag, const std::vector<double> & g,
                         const std::vector<double> & gDiag);
@@ -394,12 +397,6 @@ namespace nsfem
         int rowsDir_ = 0, rowsUpd_ = 0, rowsRho_ = 0, lanesDir_ = 0;
         BlockMap bmDir_{}, bmUpd_{}, bmRho_{};
         int nbDir_ = 0, nbUpd_ = 0, nbRho_ = 0, color0BlocksRho_ = 0;
-        // the approximate inverse's map: the direction map, or (rowsPrecond_
-        // > 0, fused reductions on one system) a region-major map of its own
-        int rowsPrecond_ = 0;
-        BlockMap bmPre_{};
-        int nbPre_ = 0;
-        DeviceArray<int2> preTable_;
         void setupKindMaps();
         // the colour sweeps' workgroup map
         int sweepLanes_ = 8, sweepRows_ = 0;

@@ -189,40 +189,42 @@ def test_captured_steps_with_fsai_velocity():
     assert st["capturedStep"] == 0 and captured.step_graph_info()["rollbacks"] == before + 1
 
 
-def test_fsai_on_a_map_of_its_own(channel_20k):
-    """rowsPreconditioner gives the approximate inverse's two launches a
-    region-major map of their own (here 256-row workgroups against the
-    direction kernel's 1,024): the same operator, so the same solution to the
-    target and the same iteration count (the r.z partial sums only regroup);
-    counts that are not multiples of 256 are rejected."""
+@pytest.mark.parametrize("nch", [2, 4])
+def test_fsai_workgroups_take_no_row_options(channel_20k, nch):
+    """Fused solves with the approximate inverse run on workgroups of their own:
+    the row options are accepted (rowsPreconditioner only in multiples of 256),
+    change no bit of the solution, and 0 is reported for the direction and
+    update kernels; back on the sweeps the counts apply again."""
     from nsfem_amd import cu
     from nsfem_amd._lib import NsfemError
     M, _ = channel_20k
     n = M.shape[0]
     rng = np.random.default_rng(47)
-    b = np.concatenate([M @ rng.uniform(-1, 1, n) for _ in range(2)])
+    b = np.concatenate([M @ rng.uniform(-1, 1, n) for _ in range(nch)])
     out = []
-    for rows_pre in (0, 256):
-        s = cu.createSolver("pcg_mixed", 2, M, 2000, 1e-10, 1)
-        s.setOption("fusedReductions", 1)
-        s.setOption("rowsDirection", 1024)
+    for rows in (0, 1024):
+        s = cu.createSolver("pcg_mixed", nch, M, 2000, 1e-10, 1)
+        s.setOption("rowsDirection", rows)
+        s.setOption("rowsUpdate", rows)
+        counts = s.kindRows()
         s.setOption("preconditioner", 1)
-        s.setOption("rowsPreconditioner", rows_pre)
+        s.setOption("rowsPreconditioner", 256 if rows else 0)
+        assert s.kindRows()[:2] == (0, 0)
         s.getRhs().upload(b)
         s.getSol().memsetZero()
         s.solve()
         out.append((s.getLastIterations(), s.getSol().download()))
         with pytest.raises(NsfemError, match="multiple of 256"):
             s.setOption("rowsPreconditioner", 100)
-    (it0, x0), (it1, x1) = out
-    assert it0 == it1
+        s.setOption("preconditioner", 0)
+        assert s.kindRows() == counts and (not rows or counts[:2] == (1024, 1024))
+    assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
     lu = spla.splu(sp.csc_matrix(M))
-    for c in range(2):
-        xd = lu.solve(b[c * n:(c + 1) * n])
-        for x in (x0, x1):
-            xc = x[c * n:(c + 1) * n]
-            assert np.linalg.norm(b[c * n:(c + 1) * n] - M @ xc) / np.linalg.norm(b[c * n:(c + 1) * n]) <= 1.01e-10
-            assert np.max(np.abs(xc - xd)) <= 1e-7 * np.max(np.abs(xd))
+    for c in range(nch):
+        bc, xc = b[c * n:(c + 1) * n], out[0][1][c * n:(c + 1) * n]
+        xd = lu.solve(bc)
+        assert np.linalg.norm(bc - M @ xc) / np.linalg.norm(bc) <= 1.01e-10
+        assert np.max(np.abs(xc - xd)) <= 1e-7 * np.max(np.abs(xd))
 
 
 def test_fsai_rejects_what_it_does_not_cover(channel_20k):
