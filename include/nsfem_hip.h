@@ -264,7 +264,9 @@ int nsfem_solver_num_colors(const nsfem_solver * s, int system, int * out);
  * tries the sweeps on lanes x {1, 2, 4} slabs of their own, then (fused
  * reductions) the direction / update / rho rows and the direction lanes, and
  * last, unless fusedReductions was set, the finalize kernels against the
- * fused reductions; it overwrites the internal work vectors, not rhs/sol.
+ * fused reductions; it overwrites the internal work vectors, not rhs/sol, and
+ * keeps the shapes of a solver whose solves run on workgroups of their own
+ * (the approximate inverse with fused reductions).
  * Solvers of 4 to 32 channels run one
  * lane per channel (lanes = numCh) and keep at most about 16k workgroups.
  * No reference counterpart (the reference's launch shapes are fixed). */

@@ -1329,6 +1329,12 @@ namespace nsfem
         {
             throw std::invalid_argument("autotuning is available for pcg solvers");
         }
+        if (ownMap())
+        {
+            // no kernel of such a solve takes any of the shapes below: the
+            // fastest would be picked by noise and apply once the sweeps run
+            return {lanes_, rowsPerBlock_};
+        }
         // The objective is one PCG iteration replayed from a captured graph,
         // as the solver runs it: kernel durations and the gaps between the
         // dependent launches.

@@ -272,7 +272,8 @@ namespace nsfem
         // {1, 2, 4, 8} times minRowsPerBlock()) and keeps the fastest shape,
         // then the sweeps' own shape over lanes x {1, 2, 4} slabs, then (fused
         // reductions) {2, 4, 8, 16} times the rows for the direction, update
-        // and rho kernels in turn; returns (lanes, rowsPerBlock).
+        // and rho kernels in turn; returns (lanes, rowsPerBlock).  Keeps
+        // every shape where the solves run on a map of their own (ownMap()).
         // Overwrites the internal work vectors (not the io vectors).
         std::pair<int, int> autotune(int reps);
 

@@ -227,6 +227,29 @@ def test_fsai_workgroups_take_no_row_options(channel_20k, nch):
         assert np.max(np.abs(xc - xd)) <= 1e-7 * np.max(np.abs(xd))
 
 
+@pytest.mark.parametrize("nch", [1, 2, 4])
+def test_autotuning_keeps_the_shapes_of_fused_fsai_solves(channel_20k, nch):
+    """No kernel of such a solve takes one, so none is picked by noise; with the
+    finalize kernels the lane-split ones run, and there is a choice again."""
+    from nsfem_amd import cu
+    M, _ = channel_20k
+    s = cu.createSolver("pcg_mixed", nch, M, 2000, 1e-10, 1)
+    s.reshape(nch if nch > 2 else 16, 320)  # rows that autotuning never picks
+    s.reshapeSweeps(nch if nch > 2 else 2, 640)
+    s.setOption("preconditioner", 1)
+    shapes = s.shape(), s.sweepShape()
+    assert s.autotune(2) == shapes[0] and (s.shape(), s.sweepShape()) == shapes
+    s.setOption("fusedReductions", 0)
+    s.autotune(2)
+    assert s.shape() != shapes[0]
+    rng = np.random.default_rng(5)
+    b = np.concatenate([M @ rng.uniform(-1, 1, M.shape[0]) for _ in range(nch)])
+    s.getRhs().upload(b)
+    s.getSol().memsetZero()
+    s.solve()
+    assert s.getLastRelRes(0) <= 1e-10
+
+
 def test_fsai_rejects_what_it_does_not_cover(channel_20k):
     from nsfem_amd import cu
     from nsfem_amd._lib import NsfemError
