@@ -1009,6 +1009,15 @@ namespace nsfem
             part(rowStart[o], rowSplit[o], rs[i]);
             part(rowSplit[o], rowStart[o + 1], split[i]);
         }
+        loc_.systemSlice.assign(1, 0);
+        for (const RowChunk & ch : loc_.chunks)
+        {
+            loc_.systemSlice.push_back(loc_.systemSlice.back() + (ch.end - ch.begin + 63) / 64);
+        }
+        if (opt_.numCh <= 2 && !slicesFit(rs, split))
+        {
+            return;
+        }
         if (col.empty())
         {
             col.push_back(0); // a diagonal matrix: keep valid pointers
@@ -1037,13 +1046,9 @@ namespace nsfem
             loc_.g32.upload(to32(gv));
             loc_.gDiag32.upload(to32(gd));
         }
-        loc_.systemSlice.assign(1, 0);
-        for (const RowChunk & ch : loc_.chunks)
-        {
-            loc_.systemSlice.push_back(loc_.systemSlice.back() + (ch.end - ch.begin + 63) / 64);
-        }
         if (opt_.numCh > 2)
         {
+            loc_.fits = true;
             return;
         }
         // Slices of 64 rows of one system, entry k of all its rows side by
@@ -1063,10 +1068,6 @@ namespace nsfem
                     {
                         const auto [b, e] = range(r0 + l);
                         width = std::max(width, e - b);
-                    }
-                    if (sc.size() + static_cast<size_t>(width + 1) * 64 > 0x7fffffffu)
-                    {
-                        throw std::invalid_argument("approximate inverse: the sliced system exceeds 32-bit indices");
                     }
                     const int at = static_cast<int>(sc.size());
                     table.push_back(int4{r0, rows, at, width});
@@ -1103,6 +1104,52 @@ namespace nsfem
         slice(loc_.a, [&](int r) { return std::pair<int, int>(rs[r], rs[r + 1]); }, av, opt_.precision != SolverPrecision::F32);
         slice(loc_.lower, [&](int r) { return std::pair<int, int>(rs[r], split[r]); }, gv, p64);
         slice(loc_.upper, [&](int r) { return std::pair<int, int>(split[r], rs[r + 1]); }, gv, p64);
+        loc_.fits = true;
+    }
+
+    // Whether slices suit the rows [rowStart[i], rowStart[i + 1]), lower parts up
+    // to rowSplit[i].  A slice is as long as its longest row, which one lane
+    // walks alone, so rows of very different length cost padding and time; such
+    // systems stay on the lane-split kernels in colour order.  us an iteration
+    // sliced / lane-split, pcg_mixed, two channels, rows of 4 entries and one
+    // long row in 1,024 (padded entries for entries): 100k rows, rows of 130 (2.4)
+    // 36.8 / 36.1, 200 (3.7) 54.9 / 48.9, 400 (5.9) 89.3 / 69.4, one of 390 in 10,000
+    // (1.7) 59.0 / 56.3 (one channel 55.4 / 46.8); 10k rows, 200 33.6 / 40.3, 400
+    // 54.6 / 51.5; 400k rows, 130 56.5 / 76.4, 400 152 / 137.
+    bool McgsSolver::slicesFit(const std::vector<int> & rowStart, const std::vector<int> & rowSplit) const
+    {
+        constexpr int kLongest = 256;
+        constexpr double kPadding = 2.5;
+        double padded = 0, entries = 0;
+        for (int part = 0; part < 3; part++)
+        {
+            long stored = 0;
+            for (const RowChunk & ch : loc_.chunks)
+            {
+                for (int r0 = ch.begin; r0 < ch.end; r0 += 64)
+                {
+                    const int rows = std::min(64, ch.end - r0);
+                    int width = 0;
+                    for (int r = r0; r < r0 + rows; r++)
+                    {
+                        const int begin = part == 2 ? rowSplit[r] : rowStart[r], end = part == 1 ? rowSplit[r] : rowStart[r + 1];
+                        width = std::max(width, end - begin);
+                        entries += end - begin;
+                    }
+                    if (width > kLongest)
+                    {
+                        return false;
+                    }
+                    padded += static_cast<double>(width) * rows;
+                    stored += 64L * width;
+                }
+            }
+            if (stored > 0x7fffffff) // the kernels' entry offsets
+            {
+                return false;
+            }
+        }
+        return padded <= kPadding * entries;
     }
 
     void McgsSolver::setupSliceMaps()

@@ -322,8 +322,9 @@ namespace nsfem
         template <typename P>
         McgsMatrix<P> fsaiView() const;
         // The approximate inverse needs no colour order: its solves run on a
-        // copy of the system with the rows of every system in locality order.
-        bool local() const { return precond_ == 1 && !opt_.restart; }
+        // copy of the system with the rows of every system in locality order
+        // (not where one or two channels' slices do not fit the rows).
+        bool local() const { return precond_ == 1 && !opt_.restart && loc_.fits; }
         // ... and, with fused reductions on one or two channels, its products
         // on slices of 64 rows (sliced_kernels.hpp)
         bool sliced() const { return local() && fused() && opt_.numCh <= 2; }
@@ -334,6 +335,7 @@ namespace nsfem
         void buildLocal(const std::vector<int> & rowStart, const std::vector<int> & rowSplit, const std::vector<int> & column,
                         const std::vector<double> & values, const std::vector<double> & diag, const std::vector<double> & g,
                         const std::vector<double> & gDiag);
+        bool slicesFit(const std::vector<int> & rowStart, const std::vector<int> & rowSplit) const;
         // f<W>() for the waves per workgroup of the sliced kernels
         template <typename F>
         void dispatchWaves(F && f) const;
@@ -475,6 +477,7 @@ namespace nsfem
         };
         struct Local
         {
+            bool fits = false; // the copy below is there
             DeviceArray<int> perm, iperm;
             DeviceMcgs<double> A64;
             DeviceMcgs<float> A32;

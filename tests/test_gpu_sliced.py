@@ -126,3 +126,41 @@ def test_sweeps_after_a_change_of_preconditioner_equal_a_fresh_solver(sizes, nam
         s.solve()
         xs.append(s.getSol().download())
     assert np.array_equal(*xs)
+
+
+def _with_long_rows(n, length, every, base):
+    """base random neighbours a row and `length` of them every `every` rows."""
+    rng = np.random.default_rng(n + length)
+    r = np.repeat(np.arange(n), base)
+    c = (r + rng.integers(1, 60, r.size)) % n
+    for i in range(every // 2, n, every):
+        far = rng.choice(np.setdiff1d(np.arange(n), [i]), length, replace=False)
+        r, c = np.concatenate([r, np.full(length, i)]), np.concatenate([c, far])
+    a = sp.coo_matrix((-rng.uniform(0.2, 1, r.size), (r, c)), shape=(n, n)).tocsr()
+    a = a + a.T
+    a.setdiag(0)
+    a.eliminate_zeros()
+    return (a + sp.diags(np.asarray(abs(a).sum(axis=1)).ravel() * 1.2 + 1)).tocsr()
+
+
+# one row of about 200 and of 290 entries, an arrow of 700, many rows of 120 in
+# short ones (padding of about 20): all but the first stay on the lane-split
+# kernels, from four channels on none does
+@pytest.mark.parametrize("args,sliced", [((4000, 190, 4000, 4), True), ((4000, 280, 4000, 4), False), ((701, 700, 701, 0), False),
+                                         ((6000, 120, 700, 0), False)])
+@pytest.mark.parametrize("name,nch", [("pcg", 1), ("pcg_mixed", 2), ("pcg_mixed", 4)])
+@pytest.mark.parametrize("batch", [False, True])
+def test_rows_too_uneven_for_slices(args, sliced, name, nch, batch):
+    m = _with_long_rows(*args)
+    mats = [m, _spd(130, 8, "sparse")] if batch else [m]
+    n = sum(a.shape[0] for a in mats)
+    rng = np.random.default_rng(13)
+    b, x0 = rng.uniform(-1, 1, nch * n), rng.uniform(-1, 1, nch * n)
+    s, x = _run(name, nch, mats, b, x0, 1, np.float64, 1e-12)
+    assert (s.kindRows()[0] == 0) == (sliced or nch > 2)
+    a = sp.block_diag(mats).tocsr()
+    for c in range(nch):
+        bc, xc = b[c * n:(c + 1) * n], x[c * n:(c + 1) * n]
+        assert np.linalg.norm(bc - a @ xc) <= 1.01e-12 * np.linalg.norm(bc) * np.sqrt(len(mats))
+    s.solve()  # from the solution: nothing left to do
+    assert np.linalg.norm(s.getSol().download() - x) <= 1e-11 * np.linalg.norm(x)
