@@ -11,7 +11,9 @@ scheme's diffusion bound (tau nu lambda_max(M^-1 K) <= 2) at this mesh size:
 the library's time-step guard (clamp policy) runs it at 1 / lambda_max(M^-1
 nu K); both values are reported.
 
-Prints one JSON line.  Progress goes to stderr."""
+Prints one JSON line, short enough for a reader that keeps only the end of a
+program's output.  The full record (every path, launch shape and kernel) goes to
+--details FILE or, without it, to stderr, as the progress does."""
 
 import argparse
 import json
@@ -26,6 +28,19 @@ sys.path.insert(0, ROOT)
 
 def log(*a):
     print(*a, file=sys.stderr, flush=True)
+
+
+LEGS = ("fp64", "mixed", "fp64_fast", "fp64_mcgs", "mixed_mcgs", "ensemble", "batch", "cpu_baseline")
+
+
+def short_record(record):
+    """The record without the kernel table, and of each leg its numbers, texts
+    and iteration counts."""
+    short = {k: v for k, v in record.items() if k != "kernels"}
+    for leg in LEGS:
+        if isinstance(record.get(leg), dict):
+            short[leg] = {k: v for k, v in record[leg].items() if k == "iters" or isinstance(v, (bool, int, float, str))}
+    return short
 
 
 def build_workload(nodes, seed, gpu_assembly=False):
@@ -625,11 +640,10 @@ def main():
     ap.add_argument("--fast-shape", default="2,256,2,512,512,4096,1024,2,1",
                     help="velocity launch shape of the fast paths (mixed, fp64_fast): lanes, rows per block, sweep "
                          "lanes, sweep rows, direction / update / rho rows, direction lanes, fused reductions, and "
-                         "optionally the approximate inverse's rows (0: the direction kernel's map); the "
-                         "measured best on MI355X (the autotuner's direction-row candidates are multiples of the base "
-                         "rows it picks first, and from a 1,024-row base miss these 512-row workgroups, 10 %% per "
-                         "iteration); 'auto' autotunes them like the other paths; an explicit "
-                         "--shape takes precedence")
+                         "optionally rowsPreconditioner (no effect); used with --velocity-precond sgs, without "
+                         "effect on the approximate inverse's solves, which take workgroups of their own; 'auto' "
+                         "autotunes them like the other paths; an explicit --shape takes precedence")
+    ap.add_argument("--details", default="", help="write the full record (JSON) to this file instead of stderr")
     ap.add_argument("--no-kernels", action="store_true", help="skip the per-kernel timing table")
     ap.add_argument("--step-graph", action="store_true",
                     help="each step as one captured graph with device-side convergence (after a first regular step)")
@@ -938,7 +952,13 @@ def main():
         "batch": batch,
         "setup_s": setup_s,
     }
-    print(json.dumps(out))
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(out, f)
+            f.write("\n")
+    else:
+        log(json.dumps(out))
+    print(json.dumps(short_record(out)))
     return 0
 
 
