@@ -42,15 +42,21 @@ def _run(name, nch, mats, b, x0, fused, dtype, target):
 
 # 64 rows are a slice; 2, 4 and 8 waves a workgroup up to 256, 1,024 and more
 # slices; a window of 1,024 rows is sorted together
-@pytest.mark.parametrize("sizes", [[1], [63], [64], [65], [1023], [1025], [257 * 64 + 1], [1025 * 64 + 5], [40, 1, 700, 64, 130]])
-@pytest.mark.parametrize("name,nch,dtype", [("pcg", 1, np.float64), ("pcg", 2, np.float64), ("pcg_mixed", 2, np.float64),
-                                            ("pcg_mixed", 1, np.float64), ("pcg", 2, np.float32), ("pcg", 4, np.float64),
-                                            ("pcg_mixed", 8, np.float64), ("pcg_mixed", 16, np.float64), ("pcg", 16, np.float32),
-                                            ("pcg", 32, np.float64)])
-@pytest.mark.parametrize("kind", ["sparse", "long", "diagonal"])
+SIZES = [[1], [63], [64], [65], [1023], [1025], [257 * 64 + 1], [1025 * 64 + 5], [40, 1, 700, 64, 130]]
+SOLVERS = [("pcg", 1, np.float64), ("pcg", 2, np.float64), ("pcg_mixed", 2, np.float64), ("pcg_mixed", 1, np.float64),
+           ("pcg", 2, np.float32), ("pcg", 4, np.float64), ("pcg_mixed", 8, np.float64), ("pcg_mixed", 16, np.float64),
+           ("pcg", 16, np.float32), ("pcg", 32, np.float64)]
+# one or two channels and one pattern reach the largest sizes; from 262,144 rows
+# on (4,096 slices) a workgroup walks its slices in more than one turn, and
+# vectors of more than 8M values take twice the workgroups
+CASES = [(kind, *solver, sizes) for kind in ("sparse", "long", "diagonal") for solver in SOLVERS for sizes in SIZES
+         if max(sizes) < 20_000 or (kind == "sparse" and solver[1] <= 2)]
+CASES += [("sparse", "pcg", 1, np.float64, [4097 * 64 + 3]), ("sparse", "pcg_mixed", 2, np.float64, [4097 * 64 + 3, 700]),
+          ("sparse", "pcg_mixed", 32, np.float64, [4097 * 64 + 3])]
+
+
+@pytest.mark.parametrize("kind,name,nch,dtype,sizes", CASES)
 def test_sliced_solves_equal_the_general_kernels(sizes, name, nch, dtype, kind):
-    if (kind != "sparse" or nch > 2) and max(sizes) > 20_000:
-        pytest.skip("one or two channels and one pattern reach the largest sizes")
     mats = [_spd(n, 100 + n, kind) for n in sizes]
     n = sum(sizes)
     rng = np.random.default_rng(7)
