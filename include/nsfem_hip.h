@@ -128,7 +128,8 @@ int nsfem_convert(int srcDtype, int dstDtype, long n, const void * src, void * d
  *                      greedy aggregation, Jacobi-smoothed prolongation,
  *                      Galerkin coarse operators until one is small enough to be inverted
  *                      densely: 5,120 rows in FP32, 3,620 in FP64, 2,432 from
- *                      four columns on) smoothed by one multicolour GS sweep per
+ *                      four columns on, 1,536 on four in FP64 directly under
+ *                      the finest level) smoothed by one multicolour GS sweep per
  *                      direction on the finest level (forward down, backward
  *                      up) and two Chebyshev steps on D^-1 A on the coarser
  *                      ones (options "amgChebyshev*" below); one system,

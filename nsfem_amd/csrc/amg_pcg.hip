@@ -1142,12 +1142,20 @@ namespace nsfem
         // the deeper levels that it replaces, some 3.3 us each.  Up to 100 MB
         // (5,120 rows in FP32, 3,620 in FP64) it stays in the Infinity Cache.
         // Measured per CG iteration against 512 rows: 60k rows FP64 78.9 ->
-        // 66.4 us, 300k FP64 (2,700 coarse rows) 120 -> 111, 500k FP32 (4,624)
+        // 66.4 us, 300k FP64 (2,700 coarse rows) 120 -> 111, 500k FP32 (4,620)
         // 129.6 -> 124.8, 100k x 16 FP32 (1,008) 170 -> 157.  Four channels or
         // more do that many times the arithmetic per entry: 40k x 8 FP32 with
-        // 4,400 coarse rows took 105 us against 89 with 432.
+        // 4,400 coarse rows took 105 us against 89 with 432.  Up to 2,432 rows, us a
+        // solve of 10k / 16k / 22k / 100k / 200k rows (1.0k, 1.65k, 2.3k, 1.0k, 1.9k
+        // coarse rows) against 512: 8 columns FP64 1,408 -> 1,226, 1,397 -> 1,386,
+        // 1,626 -> 1,594, 2,834 -> 2,588, 4,282 -> 4,102; 16 columns FP32 1,510 ->
+        // 1,247, 1,548 -> 1,426, 1,776 -> 1,605, 3,191 -> 2,709, 4,778 -> 4,468;
+        // 4 columns FP32 1,202 -> 914, 1,129 -> 959, 1,214 -> 1,145, 1,969 -> 1,661,
+        // 2,624 -> 2,327, but FP64 1,293 -> 1,016, 1,208 -> 1,262, 1,327 -> 1,575,
+        // 2,261 -> 2,024, 3,121 -> 2,997: directly under the finest level 1,536.
         constexpr long kCoarseBytes = 100L << 20;
         constexpr int kMaxCoarseWide = 2432;
+        constexpr int kMaxCoarseSecond4F64 = 1536;
     } // namespace
 
     AmgPcg::AmgPcg(const CsrD & stripped, const std::vector<int> & rowSplit, const std::vector<double> & diag,
@@ -1170,7 +1178,8 @@ namespace nsfem
             opt.maxCoarse = std::min(maxCoarse, n_ - 1);
             opt.invertCoarse = false;
             h = buildAmgHierarchy(stripped, rowSplit, diag, colorStart, opt);
-            if (h.levels.back().n <= maxCoarse)
+            const bool second4F64 = nch_ == 4 && !mixed_ && h.levels.size() == 2;
+            if (h.levels.back().n <= (second4F64 ? kMaxCoarseSecond4F64 : maxCoarse))
             {
                 coarseN_ = h.levels.back().n;
                 coarseLd_ = (coarseN_ + 63) / 64 * 64;
@@ -1189,9 +1198,9 @@ namespace nsfem
         }
         if (!inverted)
         {
-            // small systems, coarsening that stalls, and operators that are not
-            // definite on that level: down to 512 rows, inverted (or
-            // rejected) on the host
+            // small systems, a level past its limit, coarsening that stalls, and
+            // operators that are not definite on that level: down to 512 rows,
+            // inverted (or rejected) on the host
             h = buildAmgHierarchy(stripped, rowSplit, diag, colorStart);
         }
         complexity_ = h.operatorComplexity;
