@@ -29,7 +29,7 @@ namespace nsfem
 {
     // Rows of the locality order that are sorted by entry count together.
     constexpr int kSortWindow = 1024;
-    // Workgroups of a kernel at most: every one of the next kernel re-sums all
+    // Workgroups of a kernel, rounded up per system: every one of the next kernel re-sums all
     // partial sums of this one, and two of eight waves on every CU stream as
     // fast as four (2M rows: 224 and 220 us an iteration; 240k rows: the same).
     constexpr int kSliceGroups = 512;

@@ -582,8 +582,7 @@ namespace nsfem
         // work) once there are rows enough.  us per PCG iteration on 8 / 4 / 2
         // lanes: P2 rows, two channels, 7k rows 59.3 / 61.4 / 66.4, 100k 86.5 /
         // 79.3 / 81.8, 240k 120 / 109 / 113, 2M 635 / 521 / 523; P1 rows 1.9k 24.7 /
-        // 24.7 / 26.3, 25k 28.5 / 25.1 / 24.7, 60k 32.0 / 28.5 / 26.4.  A batch
-        // keeps the lanes by row length: its rows belong to systems of any size.
+        // 24.7 / 26.3, 25k 28.5 / 25.1 / 24.7, 60k 32.0 / 28.5 / 26.4.
         auto defaultLanes = [&]()
         {
             if (flat() && meanRow_ <= 8)
@@ -597,11 +596,17 @@ namespace nsfem
         // Default rows: a workgroup walks its row slabs one after another, each a
         // chain of dependent loads, so one slab for one system, whose main map
         // is widened per kernel kind (setupKindMaps; the sweeps write no partial
-        // sums, so any count goes); a batch's main map is every kernel's, and
-        // its partial sums are re-summed by every workgroup: four.  Measured
-        // against four slabs, us per PCG iteration: 2k pressure nodes velocity
-        // (two columns) 107 -> 59 and pressure 39.9 -> 24.7, 25k 128 -> 87 and
-        // 42.5 -> 28.6, 60k 170 -> 120 and 44.6 -> 32.0, 500k velocity 697 -> 635.
+        // sums, so any count goes).  Measured against four slabs, us per PCG
+        // iteration: 2k pressure nodes velocity (two columns) 107 -> 59 and
+        // pressure 39.9 -> 24.7, 25k 128 -> 87 and 42.5 -> 28.6, 60k 170 -> 120 and
+        // 44.6 -> 32.0, 500k velocity 697 -> 635; with finalize launches and in gs
+        // it pays at every size up to 2M rows, too (1.15 to 1.9 times as fast).
+        // A batch's main map is every kernel's: one slab on its eight lanes leaves
+        // more partial sums than it saves, 9 meshes of 5k to 25k nodes, pcg on
+        // two columns, 188 -> 244, 4 of 12k to 60k 206 -> 439 (gs 119 -> 97, 122
+        // -> 106).  Fewer lanes gain there, too (two lanes on one slab 130 and
+        // 146), but no rule for them over batches of any sizes was measured, so
+        // a batch keeps the lanes by row length and four slabs.
         // From eight columns on the sums that every workgroup of the next kernel
         // (or the finalize) adds up, columns x workgroups, come to outweigh the
         // chains, and one slab gives way to two and four (the sweeps keep one).
