@@ -636,7 +636,7 @@ def main():
                     help="launch shape velocityLanes,velocityRowsPerBlock,pressureLanes,pressureRowsPerBlock (0 = default), "
                          "optionally followed by the same four for the colour sweeps and then by the velocity and "
                          "pressure direction,update,rho rows, the velocity and pressure direction lanes and "
-                         "whether each fuses its reductions (18 numbers, as the JSON records them)")
+                         "whether each fuses its reductions (18 numbers, as the full record has them)")
     ap.add_argument("--fast-shape", default="2,256,2,512,512,4096,1024,2,1",
                     help="velocity launch shape of the fast paths (mixed, fp64_fast): lanes, rows per block, sweep "
                          "lanes, sweep rows, direction / update / rho rows, direction lanes, fused reductions, and "
