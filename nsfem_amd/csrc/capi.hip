@@ -208,10 +208,10 @@ namespace
 
 struct nsfem_csr
 {
-    int rows, cols, nnz, dtype;
+    int rows, cols, nnz, dtype, longest;
     DeviceArray<int> rowStart, column;
     DeviceArray<char> values;
-    CsrView view() const { return CsrView{rows, cols, nnz, rowStart.get(), column.get(), values.get(), dtype}; }
+    CsrView view() const { return CsrView{rows, cols, nnz, rowStart.get(), column.get(), values.get(), dtype, longest}; }
 };
 
 struct nsfem_solver
@@ -331,6 +331,11 @@ extern "C"
             m->cols = cols;
             m->nnz = nnz;
             m->dtype = dtype;
+            m->longest = 0;
+            for (int r = 0; r < rows; r++)
+            {
+                m->longest = std::max(m->longest, h.rowStart[r + 1] - h.rowStart[r]);
+            }
             m->rowStart.upload(h.rowStart);
             m->column.upload(nnz ? h.column : std::vector<int>{0});
             const size_t vb = std::max<size_t>(1, nnz) * dtypeSize(dtype);

@@ -81,8 +81,8 @@ namespace nsfem
                 default: throw std::invalid_argument("lanes must be 4, 8, 16, 32 or 64");
                 }
             };
-            // lanes = 0: lanesForMeanRow's shape, which suits a launch that is one
-            // latency long (short chains, many CUs), until the rows are so many
+            // lanes = 0: lanesForMeanRow's shape, also for uneven rows; it suits a
+            // launch that is one latency long (short chains, many CUs), until the rows are so many
             // that idle lanes count; then fewer lanes with more loads in flight.
             // A row count where a shape is ahead on every measured matrix of
             // its bin is the line: P1, P2, divergence and gradient matrices of
@@ -108,6 +108,11 @@ namespace nsfem
             auto byRows = [&]<int C>(const T * xs, T * ys)
             {
                 constexpr bool f64 = std::is_same_v<T, double>;
+                if (!evenRows(mean, A.longest))
+                {
+                    byLanes.template operator()<C>(lanesForMeanRow(mean), xs, ys);
+                    return;
+                }
                 if constexpr (f64)
                 {
                     if (mean >= 4 && mean < 5 && outRows >= 393216)

@@ -27,7 +27,18 @@ namespace nsfem
         const int * column;
         const void * values;
         int dtype;
+        int longest = 0; // row; 0: not known, the rows are taken as even
     };
+
+    // Whether rows are even enough for the launch shapes of few lanes a row.  A
+    // wavefront holds more rows there and ends with its longest, so matrices
+    // with rows far above the mean keep the lanes of lanesForMeanRow.  FEM rows
+    // stay below the line (P1 7 of at most 9, P2 11.5 of 25, divergence 38 of 50).
+    // Past it, one row in 1,024 that long, few lanes against those: products of
+    // 100k rows, 5 entries of at most 50 0.95 to 1.0 times as fast, 110 0.92 to
+    // 0.97, 400 0.81 to 0.87, 15 of 220 0.95, 910 0.80; PCG with the sweeps, 8 of 73
+    // 0.94, 130 0.82, 490 0.67.
+    inline bool evenRows(double mean, int longest) { return longest <= 4 * mean + 16; }
 
     // y[c*ldy + i] = alpha * sum_j A[i,j] x[c*ldx + j] + beta * y[...]
     // rowIds (optional, device): output row i is A's row rowIds[i]; outRows rows.

@@ -7,14 +7,14 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def _matrix(rows, mean, seed):
+def _matrix(rows, mean, seed, longest):
     """rows x (rows - 7) with exactly rows * mean entries (rounded down), among
-    them rows without an entry (the first and the last too) and one of 300."""
+    them rows without an entry (the first and the last too) and a longest one."""
     rng = np.random.default_rng(seed)
     total = int(rows * mean)
     count = rng.integers(max(0, int(mean * 0.5)), int(np.ceil(mean * 1.5)) + 1, rows)
     count[[0, rows // 3, rows - 1]] = 0
-    count[rows // 2] = 300
+    count[rows // 2] = longest
     free = np.setdiff1d(np.arange(1, rows - 1), [rows // 3, rows // 2])
     while (d := total - int(count.sum())) != 0:
         pick = rng.choice(free, min(abs(d), free.size), replace=False)
@@ -27,14 +27,17 @@ def _matrix(rows, mean, seed):
 
 
 # the lines: 16,384 (one latency long below), 32,768 (5 to 9 entries), 65,536 (11
-# to 12, 12 to 24, 24 to 48), 393,216 (4 to 5, FP64) rows
+# to 12, 12 to 24, 24 to 48), 393,216 (4 to 5, FP64) rows; a row longer than 4 x
+# mean + 16 keeps the general shape
 @pytest.mark.parametrize("rows,mean", [(16383, 37.5), (16385, 37.5), (16385, 30), (32767, 7), (32769, 7), (65535, 11.4), (65537, 11.4),
                                        (65535, 15), (65537, 15), (65537, 30), (393215, 4.7), (393217, 4.7),
                                        (65539, 4), (65539, 5), (65539, 9), (65539, 11), (65539, 12), (65539, 24), (65539, 48)])
+@pytest.mark.parametrize("over", [0, 1])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-def test_default_shapes(rows, mean, dtype):
+def test_default_shapes(rows, mean, dtype, over):
     from nsfem_amd import cu
-    start, column, values, row, count = _matrix(rows, mean, rows + int(10 * mean))
+    start, column, values, row, count = _matrix(rows, mean, rows + int(10 * mean), int(4 * mean + 16) + over)
+    assert count.max() == int(4 * mean + 16) + over
     cols = rows - 7
     values = values.astype(dtype)
     A = cu.csrF(rows, cols, start, column, values)
