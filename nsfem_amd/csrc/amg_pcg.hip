@@ -1126,11 +1126,20 @@ namespace nsfem
         // V-cycle: 130 us an iteration, 135 on four lanes, 159 on eight; the
         // direction kernel 15.1, 17.1 and 27.8 us).  Longer rows (the coarse
         // levels' 17 entries) measure the same on 4 to 16 lanes.
-        int levelLanes(double meanRow) { return meanRow <= 8 ? 2 : lanesFor(meanRow); }
+        int levelLanes(double meanRow, int longest) { return meanRow <= 8 && evenRows(meanRow, longest) ? 2 : lanesFor(meanRow); }
         double meanRow(const std::vector<int> & rowStart)
         {
             const int rows = static_cast<int>(rowStart.size()) - 1;
             return rows > 0 ? static_cast<double>(rowStart.back()) / rows : 1.0;
+        }
+        int longestRow(const std::vector<int> & rowStart)
+        {
+            int longest = 0;
+            for (size_t i = 0; i + 1 < rowStart.size(); i++)
+            {
+                longest = std::max(longest, rowStart[i + 1] - rowStart[i]);
+            }
+            return longest;
         }
     } // namespace
 
@@ -1214,7 +1223,7 @@ namespace nsfem
             L.n = H.n;
             L.colorStart = H.colorStart;
             L.lambdaMax = H.lambdaMax;
-            L.lanes = levelLanes(meanRow(H.stripped.rowStart));
+            L.lanes = levelLanes(meanRow(H.stripped.rowStart), longestRow(H.stripped.rowStart));
             L.nnz = H.stripped.nnz();
             for (int i = 0; i < H.n; i++)
             {

@@ -240,6 +240,10 @@ namespace nsfem
             sysRows_.push_back(layouts.back().n);
             n_ += layouts.back().n;
             nnzOff += layouts.back().stripped.nnz();
+            for (int i = 0; i < layouts.back().n; i++)
+            {
+                longestRow_ = std::max(longestRow_, layouts.back().stripped.rowStart[i + 1] - layouts.back().stripped.rowStart[i]);
+            }
             numColors_ = std::max(numColors_, layouts.back().numColors());
             colorings_.push_back(layouts.back().coloring);
             partitions_.push_back(layouts.back().partitionStart);
@@ -585,11 +589,12 @@ namespace nsfem
         // 24.7 / 26.3, 25k 28.5 / 25.1 / 24.7, 60k 32.0 / 28.5 / 26.4.
         auto defaultLanes = [&]()
         {
-            if (flat() && meanRow_ <= 8)
+            const bool few = flat() && evenRows(meanRow_, longestRow_);
+            if (few && meanRow_ <= 8)
             {
                 return n_ >= 16384 ? 2 : 4;
             }
-            return flat() && meanRow_ < 12 && n_ >= 32768 ? 4 : std::min(16, lanesForMeanRow(meanRow_));
+            return few && meanRow_ < 12 && n_ >= 32768 ? 4 : std::min(16, lanesForMeanRow(meanRow_));
         };
         const int L = opt_.numCh > 2 ? opt_.numCh : (lanes > 0 ? lanes : defaultLanes());
         const int slab = kBlock / L;

@@ -378,6 +378,7 @@ namespace nsfem
         };
         std::vector<RowChunk> chunks_;     // colour-major
         double meanRow_ = 0;               // off-diagonal entries per row
+        int longestRow_ = 0;
         int rowsPerBlock_ = 0;
         std::vector<int> colorRowStart_; // numColors + 1 (global colour-major order)
         // one system: colour c's rows split into 8 stretches of the locality

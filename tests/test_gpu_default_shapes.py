@@ -70,3 +70,28 @@ def test_default_slabs_of_wide_tiles(n, nch, slabs, name):
         bound = 1.01 * target * (np.sqrt(n * nch) if name == "gs" else np.linalg.norm(b[c]))
         bound += 8 * np.finfo(np.float64).eps * np.linalg.norm(abs(a) @ abs(x[c]))
         assert np.linalg.norm(b[c] - a @ x[c]) <= bound
+
+
+# a row of more than 4 x mean + 16 off-diagonal entries keeps the lanes by the
+# mean row length, 8 for 6 and 10 entries: fewer make wavefronts of more rows
+@pytest.mark.parametrize("half,n,lanes", [(3, 20000, 2), (5, 40001, 4)])
+@pytest.mark.parametrize("name", ["pcg", "pcg_mixed", "gs"])
+def test_default_lanes_of_uneven_rows(half, n, lanes, name):
+    from nsfem_amd import cu
+    a = _band(n, half)
+    longest = 4 * 2 * half + 16
+    rng = np.random.default_rng(6)
+    b = rng.uniform(-1, 1, n)
+    target = 1e-11
+    for extra, want in ((0, lanes), (longest - 2 * half - 2, lanes), (longest, 8)):
+        far = n // 2 + 100 + 3 * np.arange(extra)
+        e = sp.coo_matrix((np.full(extra, -0.1), (np.full(extra, n // 2), far)), shape=(n, n)).tocsr()
+        m = (a + e + e.T + sp.diags(np.asarray((abs(e) + abs(e.T)).sum(axis=1)).ravel())).tocsr()
+        s = cu.createSolver(name, 1, m, 400, target, 1)
+        assert s.shape() == (want, 256 // want), extra
+        s.getRhs().upload(b)
+        s.getSol().memsetZero()
+        s.solve()
+        x = s.getSol().download()
+        bound = 1.01 * target * (np.sqrt(n) if name == "gs" else np.linalg.norm(b)) + 8 * np.finfo(float).eps * np.linalg.norm(abs(m) @ abs(x))
+        assert np.linalg.norm(b - m @ x) <= bound
